@@ -27,7 +27,7 @@ _ref = None
 def build():
     """Compile the oracle (and, where /root/reference is present, the reference's CPU path)."""
     subprocess.run(["make", "-s", "-C", HERE], check=True)
-    if os.path.isdir("/root/reference"):
+    if os.path.isfile("/root/reference/src/cpu/q8.c"):
         subprocess.run(["make", "-s", "-C", HERE, "ref"], check=True)
 
 
