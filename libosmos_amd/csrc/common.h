@@ -105,7 +105,11 @@ __device__ inline T* table_at(T* const* tab, uint32_t i) {
 }
 template <typename V>
 __device__ inline V gload(const void* p) {
+#if __HIP_DEVICE_COMPILE__
   return *(const __attribute__((address_space(1))) V*) p;
+#else
+  return *(const V*) p;  // (the host pass only parses this; a struct there has no copy from an address space)
+#endif
 }
 __device__ inline uint32_t ld32(const uint8_t* p) { return ld16(p) | ld16(p + 2) << 16; }
 __device__ inline float f16(uint32_t bits) { return __half2float(__ushort_as_half((unsigned short) bits)); }

@@ -7,12 +7,13 @@
 // matrix-core steps from zero each, then the partitions summed in order. a token's sums its own: the same bits at any
 // batch, tiling or grouping.
 //
-// CDNA4 mapping: a workgroup is 16 rows x W waves, wave p partition p; each step is v_mfma_f32_16x16x32_f16 (32
-// values: the gfx950 f16 MMA's K, the reference's WMMA takes 16) - A the lane's row's 8 decoded values, B the same 8
-// columns of its token.
+// CDNA4 mapping: each step is v_mfma_f32_16x16x32_f16 (32 values: the gfx950 f16 MMA's K, the reference's WMMA takes
+// 16) - A the lane's row's 8 decoded values, B the same 8 columns of its token. Q4_0, Q3_K, Q4_K, IQ1_S, IQ1_M, IQ2_XXS and
+// IQ3_XXS decode straight from global memory (split_kernel, rows_kernel; mmraw.h); the other types, and a Q4_0 width that
+// is not whole 256s, stage their rows in LDS (kernel: a workgroup 16 rows x W waves, wave p partition p).
 #include <type_traits>
 
-#include "decode.h"
+#include "mmraw.h"
 #include "x16.h"
 
 extern "C" {
@@ -23,10 +24,6 @@ namespace osm {
 namespace mm {
 
 __constant__ DecodeTables kDec = make_decode_tables();
-
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kTile = kX16Tile, kStep = 32;
 
@@ -41,28 +38,19 @@ struct Args {
   float* y;
 };
 
-// the IQ2 / IQ3 grids as f16 (each grid byte's value as f16 bits) and the 8-value sign masks as f16 sign bits
+// the IQ2_XS and IQ2_S grids as f16 (each grid byte's value as f16 bits) and the 8-value sign masks as f16 sign bits
 // (0x8000 in each negated value): sign7 by a 7-bit sign index (its parity bit folded in, gguf's ksigns), sign8 by
 // the 8 sign bits themselves
-constexpr uint16_t half_bits(uint32_t n) {  // a small positive integer's f16 bits
-  int e = 0;
-  while ((n >> (e + 1)) != 0) e++;
-  return (uint16_t) ((15 + e) << 10 | ((n << (10 - e)) & 0x3FFu));
-}
 struct alignas(16) HalfGrids {
-  uint16_t iq2xxs[256][8], iq2xs[512][8], iq2s[1024][8], iq3xxs[256][4], sign7[128][8], sign8[256][8];
+  uint16_t iq2xs[512][8], iq2s[1024][8], sign7[128][8], sign8[256][8];
 };
 constexpr HalfGrids make_half_grids() {
   const Grids g = make_grids();
   HalfGrids h{};
-  for (int i = 0; i < 256; i++)
-    for (int j = 0; j < 8; j++) h.iq2xxs[i][j] = half_bits((uint32_t) (g.iq2xxs[i] >> (8 * j)) & 0xFF);
   for (int i = 0; i < 512; i++)
     for (int j = 0; j < 8; j++) h.iq2xs[i][j] = half_bits((uint32_t) (g.iq2xs[i] >> (8 * j)) & 0xFF);
   for (int i = 0; i < 1024; i++)
     for (int j = 0; j < 8; j++) h.iq2s[i][j] = half_bits((uint32_t) (g.iq2s[i] >> (8 * j)) & 0xFF);
-  for (int i = 0; i < 256; i++)
-    for (int j = 0; j < 4; j++) h.iq3xxs[i][j] = half_bits((g.iq3xxs[i] >> (8 * j)) & 0xFF);
   for (int i = 0; i < 256; i++) {
     int par = 0;
     for (int j = 0; j < 7; j++) par ^= (i >> j) & 1;
@@ -77,14 +65,10 @@ constexpr HalfGrids make_half_grids() {
 __constant__ HalfGrids kHalf = make_half_grids();
 
 // the codebook a type's decoder reads, held in LDS: for the generic decoder (decode.h's Layout<T>::at `tables`) only
-// the members that type reads; for the f16 path of the IQ2 / IQ3 types (decode_h below) the f16 grid and sign masks
+// the members that type reads; for the f16 path of IQ2_XS and IQ2_S (decode_h below) the f16 grid and sign masks
 template <uint32_t T> struct LdsTab { struct { } g; };
-template <> struct LdsTab<kIQ2_XXS> { uint16_t grid[256][8], sign[128][8]; };
 template <> struct LdsTab<kIQ2_XS> { uint16_t grid[512][8], sign[128][8]; };
 template <> struct LdsTab<kIQ2_S> { uint16_t grid[1024][8], sign[256][8]; };
-template <> struct LdsTab<kIQ3_XXS> { uint16_t grid[256][4], sign[128][8]; };
-template <> struct LdsTab<kIQ1_S> { struct { uint64_t iq1s[2048]; } g; };
-template <> struct LdsTab<kIQ1_M> { struct { uint64_t iq1s[2048]; } g; };
 template <> struct LdsTab<kIQ4_NL> { struct { } g; alignas(4) int8_t iq4nl[16]; };
 template <> struct LdsTab<kIQ4_XS> { struct { } g; alignas(4) int8_t iq4nl[16]; };
 
@@ -95,68 +79,38 @@ __device__ inline void fill_tab(LdsTab<T>& t) {  // every thread of the workgrou
   uint32_t words = 0, words2 = 0;
   uint32_t* dst = (uint32_t*) &t;
   uint32_t* dst2 = nullptr;
-  if constexpr (T == kIQ2_XXS || T == kIQ2_XS || T == kIQ2_S || T == kIQ3_XXS) {
-    if constexpr (T == kIQ2_XXS) src = (const uint32_t*) kHalf.iq2xxs;
-    else if constexpr (T == kIQ2_XS) src = (const uint32_t*) kHalf.iq2xs;
-    else if constexpr (T == kIQ2_S) src = (const uint32_t*) kHalf.iq2s;
-    else src = (const uint32_t*) kHalf.iq3xxs;
+  if constexpr (T == kIQ2_XS || T == kIQ2_S) {
+    src = T == kIQ2_XS ? (const uint32_t*) kHalf.iq2xs : (const uint32_t*) kHalf.iq2s;
     src2 = T == kIQ2_S ? (const uint32_t*) kHalf.sign8 : (const uint32_t*) kHalf.sign7;
     words = sizeof t.grid / 4, words2 = sizeof t.sign / 4, dst = (uint32_t*) t.grid, dst2 = (uint32_t*) t.sign;
-  } else if constexpr (T == kIQ1_S || T == kIQ1_M) src = (const uint32_t*) kDec.g.iq1s, words = sizeof t / 4;
+  }
   else if constexpr (T == kIQ4_NL || T == kIQ4_XS) src = (const uint32_t*) kDec.iq4nl, words = 4, dst = (uint32_t*) t.iq4nl;
   for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) dst[i] = src[i];
   for (uint32_t i = threadIdx.x; i < words2; i += blockDim.x) dst2[i] = src2[i];
 }
 
-// the IQ2 / IQ3 types straight to f16: their values are (scale) x (+-grid byte) with the product exact in F32
-// (scale d (0.5 + s) / 4 or / 2: at most 16 significant bits; a grid byte at most 6), so each value is the f16 grid
-// byte, its sign bit xored in, times the F32 scale and rounded once to f16 - decode.h's exact value rounded to f16,
-// the same bits, with no integer-to-float step
+// IQ2_XS and IQ2_S straight to f16: their values are (scale) x (+-grid byte) with the product exact in F32 (scale
+// d (0.5 + s) / 4: at most 16 significant bits; a grid byte at most 6), so each value is the f16 grid byte, its sign bit
+// xored in, times the F32 scale and rounded once to f16 - decode.h's exact value rounded to f16, the same bits
 template <uint32_t T>
 constexpr bool half_path() {
-  return T == kIQ2_XXS || T == kIQ2_XS || T == kIQ2_S || T == kIQ3_XXS;
+  return T == kIQ2_XS || T == kIQ2_S;
 }
 template <uint32_t T>
 __device__ inline half8 decode_h(const LdsTab<T>& t, const uint8_t* b, int k) {
   uint4 g, sg;
-  float scale;
-  if constexpr (T == kIQ2_XXS) {
-    const uint8_t* g8 = b + 2 + 8 * (k >> 2);
-    const uint32_t aux = ld32(g8 + 4);
-    scale = mul(mul(half_at(b), 0.5f + (float) (aux >> 28)), 0.25f);
-    g = *(const uint4*) t.grid[g8[k & 3]], sg = *(const uint4*) t.sign[(aux >> (7 * (k & 3))) & 127u];
-  } else if constexpr (T == kIQ2_XS) {
-    const uint32_t e = ld16(b + 2 + 2 * k), s = (b[66 + (k >> 2)] >> (4 * ((k >> 1) & 1))) & 15u;
-    scale = mul(mul(half_at(b), 0.5f + (float) s), 0.25f);
+  uint32_t s;
+  if constexpr (T == kIQ2_XS) {
+    const uint32_t e = ld16(b + 2 + 2 * k);
+    s = (b[66 + (k >> 2)] >> (4 * ((k >> 1) & 1))) & 15u;
     g = *(const uint4*) t.grid[e & 511u], sg = *(const uint4*) t.sign[e >> 9];
-  } else if constexpr (T == kIQ2_S) {
-    const uint32_t s = (b[74 + (k >> 2)] >> (4 * ((k >> 1) & 1))) & 15u;
+  } else {
     const uint32_t idx = b[2 + k] | ((b[66 + (k >> 2)] >> (2 * (k & 3))) & 3u) << 8;
-    scale = mul(mul(half_at(b), 0.5f + (float) s), 0.25f);
+    s = (b[74 + (k >> 2)] >> (4 * ((k >> 1) & 1))) & 15u;
     g = *(const uint4*) t.grid[idx], sg = *(const uint4*) t.sign[b[34 + k]];
-  } else {  // IQ3_XXS: two 4-value grid entries a chunk
-    const uint8_t* idx = b + 2 + 2 * k;
-    const uint32_t aux = ld32(b + 66 + 4 * (k >> 2));
-    scale = mul(mul(half_at(b), 0.5f + (float) (aux >> 28)), 0.5f);
-    const uint2 g0 = *(const uint2*) t.grid[idx[0]], g1 = *(const uint2*) t.grid[idx[1]];
-    g = uint4{g0.x, g0.y, g1.x, g1.y}, sg = *(const uint4*) t.sign[(aux >> (7 * (k & 3))) & 127u];
   }
   const uint32_t w[4] = {g.x ^ sg.x, g.y ^ sg.y, g.z ^ sg.z, g.w ^ sg.w};
-  // each word's two values times the scale, rounded to f16 into the low and the high half of one register (the mixed
-  // fma: an F32 and an f16 operand, exact product, plus -0 so that a -0 product stays -0, one rounding to f16; the
-  // low form keeps the high half and the high form the low one, so the pair needs no packing)
-  uint32_t p[4];
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-#if __HIP_DEVICE_COMPILE__  // (the instruction exists on the device only; the host pass never runs this)
-    asm("v_fma_mixlo_f16 %0, %1, %2, neg(0) op_sel_hi:[0,1,0]\n\t"
-        "v_fma_mixhi_f16 %0, %1, %2, neg(0) op_sel:[0,1,0] op_sel_hi:[0,1,0]"
-        : "=&v"(p[i])
-        : "v"(scale), "v"(w[i]));
-#else
-    p[i] = w[i] ^ __float_as_uint(scale);
-#endif
-  return __builtin_bit_cast(half8, u32x4{p[0], p[1], p[2], p[3]});
+  return scaled8(mul(mul(half_at(b), 0.5f + (float) s), 0.25f), w);
 }
 
 // a type's K split (reference kernels/mm.hip:24-73, the Tuned / Short / Odd shapes): SL values a slab, W partitions.
@@ -196,10 +150,7 @@ template <uint32_t T> KSplit shape_of(uint32_t cols, bool group) {
 // slots with the same columns, so each step is its 32 values' dot product whatever order the unit takes them in.
 // then the partitions' tiles are summed in order through LDS. RT and CT are the tiling alone: the same sums
 template <uint32_t T, uint32_t SL, int W, int CT, int RT, int WB>
-// (IQ2_XXS on 4-byte staging words held to 128 VGPRs, 4 waves a SIMD: config 5's gate 761-783 -> 733 us, no spills;
-// the other instances spill at that budget)
-__global__ __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(T == kIQ2_XXS && WB == 4 ? 4 : 1)))
-void kernel(Args a) {
+__global__ __launch_bounds__(W * kWave) void kernel(Args a) {
   typedef typename std::conditional<WB == 4, uint32_t, uint16_t>::type word;
   constexpr int kThreads = W * kWave;
   constexpr uint32_t kRows = kTile * RT;                                // the workgroup's rows
@@ -273,8 +224,8 @@ void kernel(Args a) {
   // the activations of the wave's next step (its 32 columns of each token tile), loaded a step ahead: every load made
   // (a tile past the live ones reads tile 0 again, a step past the matrix this step's columns), so the loads in flight
   // are counted exactly and each wait is for that one
-  // (not for the shapes whose registers it would spill: Q8_0's and Q4_K's four row tiles by two token tiles)
-  constexpr bool kXPre = !(RT == 4 && CT == 2 && (T == kQ8_0 || T == kQ4_K));
+  // (not for the shape whose registers it would spill: Q8_0's four row tiles by two token tiles)
+  constexpr bool kXPre = !(RT == 4 && CT == 2 && T == kQ8_0);
   half8 bn[CT];
   auto xload = [&](uint32_t kk) __attribute__((always_inline)) {
 #pragma unroll
@@ -352,6 +303,251 @@ void kernel(Args a) {
     }
 }
 
+// ---- the direct kernels: the types of mmraw.h, decoded from global memory with no staging ----
+//
+// What bounded the staged kernel: every 8-value chunk took about 9 narrow LDS reads, the codes' rows conflicting, and a
+// barrier a round; one 16-token tile of 200 experts (7168 x 2048, us, staged -> rows_kernel): Q4_K 1020 -> 490, Q3_K
+// 1406 -> 487, Q4_0 733 -> 436, IQ3_XXS 530 -> 447, IQ2_XXS 456 -> 389, IQ1_M 574 -> 370, IQ1_S 467 -> 340 (the last four
+// 2048 x 7168), Q4_K 275 us by its bytes, 290 by its decode's VALU cycles. 16-32 tokens of 40 experts: Q4_K 258 -> 140;
+// one matrix at 1999 tokens: Q4_K 320 -> 136, Q4_0 206 -> 117, IQ2_XXS 254 -> 112.
+
+// this launch's matrix and tokens
+struct Job {
+  const uint8_t* w;
+  const _Float16* x16;
+  float* y;
+  uint32_t n;
+};
+__device__ inline Job job_of(const Args& a) {
+  if (!a.wt) return Job{a.w0, a.x16, a.y, a.n};
+  const uint32_t m = blockIdx.y;
+  return Job{table_at(a.wt, m), a.x16 + a.xoff[m], a.y + a.yoff[m], (uint32_t) a.cnt[m]};
+}
+// bytes of a row's 256 values
+template <uint32_t T> constexpr uint32_t span() { return 256 / Block<T>::values * Block<T>::bytes; }
+// the four output rows a lane holds of a tile, r .. r + 3 of token t
+__device__ inline void store4(float* y, uint32_t ys, uint32_t t, uint32_t n, uint32_t r, uint32_t rows, f32x4 s) {
+  if (t >= n || r >= rows) return;  // (rows a multiple of 16: all four or none)
+  float* o = y + (uint64_t) t * ys + r;
+#pragma unroll
+  for (int i = 0; i < 4; i++) o[i] = s[i];
+}
+__device__ inline f32x4 add4(f32x4 a, f32x4 b) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) a[i] = __fadd_rn(a[i], b[i]);
+  return a;
+}
+
+// a wave: RT row tiles x CT token tiles over NPW of the K split's partitions - NPW consecutive ones of every NB-th
+// 256-value block; KW waves hold them all, RW row groups of them a workgroup. a block's words are loaded while the block
+// before is decoded, x a step or more ahead (D steps), and nothing is shared until the end, where the waves add their
+// partitions in order, each onto the sums of the waves before it. few partitions a wave: many waves for a small launch;
+// a whole block's, and more rows and tokens: its decode and its x serve more products (x, not the weights, is most of
+// what a large launch reads)
+template <uint32_t T, int NPW, int RT, int CT, int RW, int D>
+__global__ __launch_bounds__(Raw<T>::W / NPW * RW * kWave) void split_kernel(Args a) {
+  using X = Raw<T>;
+  constexpr int KW = X::W / NPW, SS = X::SL / 32, NS = NPW * SS;  // partition waves, steps a slab, the wave's steps a block
+  constexpr int PB = X::NP / NPW, NB = X::W / X::NP;              // waves a block, block classes
+  __shared__ f32x4 part[KW > 1 ? RW * RT * CT * kWave : 1];
+  __shared__ Tab<T> tab;
+  const Job J = job_of(a);
+  const uint32_t t0 = blockIdx.z * kTile * CT;
+  if (t0 >= J.n) return;  // (uniform: the whole workgroup)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const int kw = wave % KW, rg = wave / KW, q = lane / 16, pw = kw % PB * NPW;
+  const uint32_t row0 = (blockIdx.x * RW + rg) * kTile * RT;
+  const int tiles = min((int) ((J.n - t0 + kTile - 1) / kTile), CT);
+  const uint32_t rb = (uint32_t) row_bytes<T>(a.cols), nblk = a.cols / 256, blk0 = kw / PB;
+  const uint8_t* wr[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; rt++)  // (rows past the matrix: its last, not stored)
+    wr[rt] = J.w + (uint64_t) min(row0 + rt * kTile + lane % 16, a.rows - 1) * rb;
+  f32x4 acc[NPW][RT][CT];
+#pragma unroll
+  for (int j = 0; j < NPW; j++)
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+      for (int ct = 0; ct < CT; ct++) acc[j][rt][ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const _Float16* xb = J.x16 + x16_at(t0 + lane % 16, 8 * q, a.xts) + (uint64_t) pw * X::SL / 16 * 256;
+  fill_step_tab<T>(tab);
+  if constexpr (Tab<T>::kSome) __syncthreads();
+  auto loop = [&](auto sub) __attribute__((always_inline)) {  // sub: the wave's part of a block, known to the compiler
+    constexpr int J0 = decltype(sub)::value * NPW;
+    uint32_t blk = blk0;
+    typename X::template R<NPW> raw[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++) X::template load<NPW>(raw[rt], wr[rt] + (uint64_t) blk * span<T>(), pw, q);
+    half8 bq[D][CT];
+    auto xload = [&](half8* b, uint32_t bl, int st) __attribute__((always_inline)) {
+#pragma unroll
+      for (int ct = 0; ct < CT; ct++)  // (a tile past the live ones reads tile 0 again)
+        b[ct] = gload<half8>(xb + (uint64_t) (ct < tiles ? ct : 0) * kTile * a.xts + (uint64_t) bl * 4096 + st * 512);
+    };
+#pragma unroll
+    for (int d = 0; d < D; d++) xload(bq[d], blk, d);
+    for (;;) {
+      const uint32_t nb = blk + NB < nblk ? blk + NB : blk;  // (past the last: it again, not used)
+      typename X::template H<NPW> h[RT];
+#pragma unroll
+      for (int rt = 0; rt < RT; rt++) X::template head<NPW>(h[rt], raw[rt], pw, q);
+#pragma unroll
+      for (int rt = 0; rt < RT; rt++) X::template load<NPW>(raw[rt], wr[rt] + (uint64_t) nb * span<T>(), pw, q);
+#pragma unroll
+      for (int st = 0; st < NS; st++) {
+        half8 av[RT], bc[CT];
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) av[rt] = X::template step<NPW>(h[rt], tab, J0 + st / SS, st % SS, q);
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++) bc[ct] = bq[st % D][ct];
+        xload(bq[st % D], st + D < NS ? blk : nb, (st + D) % NS);
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++)
+          if (ct < tiles)  // (uniform)
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++)
+              acc[st / SS][rt][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[rt], bc[ct], acc[st / SS][rt][ct], 0, 0, 0);
+      }
+      if (blk + NB >= nblk) break;
+      blk += NB;
+    }
+  };
+  if (blk0 < nblk) {  // (a row of fewer blocks than classes: this wave's partitions are empty)
+    if constexpr (X::kPart || PB == 1) {
+      loop(std::integral_constant<int, 0>{});
+    } else {
+      static_assert(PB == 2, "two waves a block");
+      if (kw % 2 == 0) loop(std::integral_constant<int, 0>{});
+      else loop(std::integral_constant<int, 1>{});
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < KW; k++) {
+    if (kw == k) {
+#pragma unroll
+      for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++) {
+          if (ct >= tiles) break;
+          const int at = ((rg * RT + rt) * CT + ct) * kWave + lane;
+          f32x4 s = k == 0 ? acc[0][rt][ct] : add4(part[at], acc[0][rt][ct]);
+#pragma unroll
+          for (int j = 1; j < NPW; j++) s = add4(s, acc[j][rt][ct]);
+          if (k + 1 < KW) part[at] = s;
+          else store4(J.y, a.ys, t0 + ct * kTile + lane % 16, J.n, row0 + rt * kTile + 4 * q, a.rows, s);
+        }
+    }
+    if (k + 1 < KW) __syncthreads();
+  }
+}
+
+// 16 tokens at most and rows enough for the chip: a wave is one row tile over all of K, every partition's sums in its
+// registers (Q4_K: 16 of 4), so nothing meets at the end; the workgroup's RW waves share x through LDS, kXCols columns at
+// a time, double-buffered. the decode of a row is then the kernel's work (one matrix instruction a decoded chunk)
+constexpr uint32_t kXCols = 256;
+template <uint32_t T, int RW>
+__global__ __launch_bounds__(RW * kWave) void rows_kernel(Args a) {
+  using X = Raw<T>;
+  constexpr int SS = X::SL / 32, NP = X::NP, W = X::W, NB = W / NP, kThreads = RW * kWave;
+  constexpr uint32_t kWords = kXCols * 2, XP = kWords / kThreads;  // 16-byte words of x a stage, and a thread
+  static_assert(kWords % kThreads == 0, "");
+  __shared__ u32x4 xs[2][kWords];
+  __shared__ Tab<T> tab;
+  const Job J = job_of(a);
+  if (!J.n) return;  // (uniform)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, q = lane / 16;
+  const uint32_t nblk = a.cols / 256, row0 = (blockIdx.x * RW + wave) * kTile;
+  const uint8_t* wr = J.w + (uint64_t) min(row0 + lane % 16, a.rows - 1) * (uint32_t) row_bytes<T>(a.cols);
+  typename X::template R<NP> raw;
+  X::template load<NP>(raw, wr, 0, q);
+  u32x4 xr[XP];
+  auto xload = [&](uint32_t blk) __attribute__((always_inline)) {
+#pragma unroll
+    for (uint32_t u = 0; u < XP; u++) xr[u] = gload<u32x4>(J.x16 + (uint64_t) blk * 4096 + (u * kThreads + threadIdx.x) * 8);
+  };
+  auto xstore = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (uint32_t u = 0; u < XP; u++) xs[buf][u * kThreads + threadIdx.x] = xr[u];
+  };
+  xload(0);
+  xstore(0);
+  fill_step_tab<T>(tab);
+  __syncthreads();
+  f32x4 acc[W];
+#pragma unroll
+  for (int j = 0; j < W; j++) acc[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  int buf = 0;
+  for (uint32_t b0 = 0; b0 < nblk; b0 += NB) {
+#pragma unroll
+    for (int sb = 0; sb < NB; sb++) {
+      const uint32_t blk = b0 + sb;
+      if (blk >= nblk) break;  // (uniform)
+      const uint32_t nb = blk + 1 < nblk ? blk + 1 : blk;
+      xload(nb);
+      typename X::template H<NP> h;
+      X::template head<NP>(h, raw, 0, q);
+      X::template load<NP>(raw, wr + (uint64_t) nb * span<T>(), 0, q);
+      const _Float16* bp = (const _Float16*) xs[buf] + q / 2 * 256 + lane % 16 * 16 + q % 2 * 8;
+#pragma unroll
+      for (int st = 0; st < 8; st++) {
+        const half8 av = X::template step<NP>(h, tab, st / SS, st % SS, q);
+        acc[sb * NP + st / SS] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, *(const half8*) (bp + st * 512), acc[sb * NP + st / SS], 0, 0, 0);
+      }
+      xstore(buf ^ 1);  // (its last reads were before the barrier before)
+      __syncthreads();
+      buf ^= 1;
+    }
+  }
+  f32x4 s = acc[0];
+#pragma unroll
+  for (int j = 1; j < W; j++) s = add4(s, acc[j]);
+  store4(J.y, a.ys, lane % 16, J.n, row0 + 4 * q, a.rows, s);
+}
+
+// the direct kernels' forms by launch size: `tiles` row tiles x matrices x token passes. a small launch splits K over as
+// many waves as the type's blocks allow (kSplit partitions a wave), a large one gives a wave a whole block's partitions
+// and two row tiles. measured, us, split / whole: one 16-token tile, Q4_K 7168 x 2048: 896 row tiles 9.3 / 12.2, 1792
+// 15.9 / 14.0; IQ2_XXS 2048 x 7168: 1024 28.0 / 32.2, 2048 50.3 / 41.3. two: Q4_K 896 11.3 / 9.9, IQ2_XXS 512 18.0 / 29.4,
+// 1024 33.3 / 30.0. four: Q4_K 448 9.2 / 8.3, IQ3_XXS 384 24.1 / 23.2, Q3_K 448 10.6 / 13.8, 896 18.3 / 13.8, IQ2_XXS 512
+// 26.0 / 36.6
+template <uint32_t T> constexpr int split_of() {
+  return T == kQ4_K ? 4 : T == kQ4_0 || T == kQ3_K || T == kIQ3_XXS ? 2 : 1;
+}
+constexpr uint64_t kLarge1 = 2048, kLarge2 = 896;
+template <uint32_t T> constexpr uint64_t large4() { return T == kQ4_K || T == kIQ3_XXS ? 384 : 768; }
+
+template <uint32_t T, int NPW, int RT, int CT, int RW, int D>
+bool launch_split(const Args& a, uint32_t n_mat, uint32_t max_n, hipStream_t s) {
+  constexpr uint32_t rows = kTile * RT * RW;
+  const dim3 grid((a.rows + rows - 1) / rows, n_mat, (max_n + kTile * CT - 1) / (kTile * CT));
+  split_kernel<T, NPW, RT, CT, RW, D><<<grid, Raw<T>::W / NPW * RW * kWave, 0, s>>>(a);
+  return hipGetLastError() == hipSuccess;
+}
+template <uint32_t T>
+bool launch_direct(const Args& a, uint32_t n_mat, uint32_t max_n, hipStream_t s) {
+  constexpr int S = split_of<T>(), NP = Raw<T>::NP;
+  const uint64_t tiles = (uint64_t) (a.rows / kTile) * n_mat;
+  if (max_n <= kTile) {
+    if (tiles < kLarge1) return launch_split<T, S, 1, 1, 1, 4>(a, n_mat, max_n, s);
+    constexpr int RW = sizeof(Tab<T>) > 16384 ? 8 : 4;  // (IQ1's 32 KB codebook: more waves a copy)
+    rows_kernel<T, RW><<<dim3((a.rows + kTile * RW - 1) / (kTile * RW), n_mat), RW * kWave, 0, s>>>(a);
+    return hipGetLastError() == hipSuccess;
+  }
+  if (max_n <= 2 * kTile) {
+    if (tiles < kLarge2) return launch_split<T, S, 1, 2, 1, 2>(a, n_mat, max_n, s);
+    return launch_split<T, NP, 2, 2, 2, 2>(a, n_mat, max_n, s);
+  }
+  if (tiles * ((max_n + 4 * kTile - 1) / (4 * kTile)) < large4<T>()) return launch_split<T, S, 1, 4, 1, 2>(a, n_mat, max_n, s);
+  // (Q4_K's whole block and IQ3_XXS's four classes would spill at two row groups or eight partitions)
+  if constexpr (T == kQ4_K) return launch_split<T, 4, 2, 4, 1, 2>(a, n_mat, max_n, s);
+  else if constexpr (T == kIQ3_XXS) return launch_split<T, NP, 2, 4, 1, 2>(a, n_mat, max_n, s);
+  else return launch_split<T, NP, 2, 4, 2, 1>(a, n_mat, max_n, s);
+}
+template <uint32_t T> constexpr bool direct() {
+  return T == kQ4_0 || T == kQ3_K || T == kQ4_K || T == kIQ1_S || T == kIQ1_M || T == kIQ2_XXS || T == kIQ3_XXS;
+}
+
 // F32 rows to the tiled f16: a thread 8 columns of one token (16 bytes out); rows at or past n zero. Rows: token t is
 // row idx[t] of x (-1: zero), read as two float4s
 template <bool Rows>
@@ -399,9 +595,8 @@ constexpr uint32_t col_tiles(uint32_t n) {
 }
 
 // token tiles a workgroup at most: 2 for a 128-value slab's shapes, 4 for the others. at 8 the 128-value shapes need
-// more than 256 VGPRs (the 128 x 8 of Q8_0 / Q6_K / IQ3_XXS spills, the 128 x 4 of IQ1 / IQ2 runs a wave a SIMD);
-// measured on 2048 -> 7168 at 512 tokens (us, caps 8 / 4 / 2): IQ3_XXS 692 / 147 / 81, IQ2_XXS 318 / 105 / 74,
-// Q8_0 704 / 144 / 104, Q4_K 83 / 69 / 96, Q4_0 88 / 59 / 72, IQ4_XS 88 / 57 / 65. the 128 x 8 shape on 2-byte
+// more than 256 VGPRs (the 128 x 8 of Q8_0 / Q6_K spills, the 128 x 4 of IQ2_XS / IQ2_S runs a wave a SIMD);
+// measured on 2048 -> 7168 at 512 tokens (us, caps 8 / 4 / 2): Q8_0 704 / 144 / 104, IQ4_XS 88 / 57 / 65. the 128 x 8 shape on 2-byte
 // staging words also spills at 4 row tiles (Q8_0 / Q6_K), so it takes one
 template <uint32_t SL> constexpr int ct_max() { return SL == 128 ? 2 : 4; }
 template <uint32_t SL, int W> constexpr bool heavy() { return SL == 128 && W == 8; }
@@ -413,7 +608,7 @@ bool launch_s(const Args& a, uint32_t n_mat, uint32_t max_n, hipStream_t s) {
   constexpr uint32_t rbr = SL * W / Block<T>::values * Block<T>::bytes;
   if (row_bytes<T>(a.cols) % 4 == 0 && rbr % 4 == 0)
     kernel<T, SL, W, CT, RT, 4><<<grid, W * kWave, 0, s>>>(a);
-  else if constexpr (RT == 1 || !heavy<SL, W>() || T == kIQ3_XXS)  // (launch_ct never takes the others)
+  else if constexpr (RT == 1 || !heavy<SL, W>())  // (launch_ct never takes the others)
     kernel<T, SL, W, CT, RT, 2><<<grid, W * kWave, 0, s>>>(a);
   else
     return false;
@@ -426,7 +621,7 @@ template <uint32_t T, uint32_t SL, int W>
 bool launch_ct(const Args& a, uint32_t n_mat, uint32_t max_n, hipStream_t s) {
   constexpr uint32_t rbr = SL * W / Block<T>::values * Block<T>::bytes;
   const bool words2 = row_bytes<T>(a.cols) % 4 != 0 || rbr % 4 != 0;
-  const bool tall = (uint64_t) n_mat * (a.rows / 64) >= 1024 && !(heavy<SL, W>() && T != kIQ3_XXS && words2);
+  const bool tall = (uint64_t) n_mat * (a.rows / 64) >= 1024 && !(heavy<SL, W>() && words2);
   const uint32_t ct = col_tiles(max_n);
   if (tall) {
     if (ct == 1) return launch_s<T, SL, W, 1, 4>(a, n_mat, max_n, s);
@@ -453,11 +648,18 @@ template <uint32_t T>
 bool run_by(const Args& a, uint32_t n_mat, uint32_t max_n, hipStream_t s) {
   const bool group = a.wt != nullptr;
   if (!fits_shape<T>(a.rows, a.cols, group)) return false;
-  const KSplit k = shape_of<T>(a.cols, group);
   constexpr KSplit t = tuned<T>(), sh = short_shape<T>(), od = odd_shape<T>();
-  if (k.sl == t.sl && k.w == t.w) return launch_ct<T, t.sl, (int) t.w>(a, n_mat, max_n, s);
-  if (k.sl == sh.sl && k.w == sh.w) return launch_ct<T, sh.sl, (int) sh.w>(a, n_mat, max_n, s);
-  return launch_ct<T, od.sl, (int) od.w>(a, n_mat, max_n, s);
+  if constexpr (direct<T>()) {
+    static_assert(t.sl == Raw<T>::SL && t.w == Raw<T>::W && sh.sl == t.sl && od.sl == t.sl, "the direct kernels' split");
+    if (a.cols % 256 == 0) return launch_direct<T>(a, n_mat, max_n, s);
+    if constexpr (T != kQ4_0) return false;  // (not reached: whole blocks of 256)
+  }
+  if constexpr (!direct<T>() || T == kQ4_0) {
+    const KSplit k = shape_of<T>(a.cols, group);
+    if (k.sl == t.sl && k.w == t.w) return launch_ct<T, t.sl, (int) t.w>(a, n_mat, max_n, s);
+    if (k.sl == sh.sl && k.w == sh.w) return launch_ct<T, sh.sl, (int) sh.w>(a, n_mat, max_n, s);
+    return launch_ct<T, od.sl, (int) od.w>(a, n_mat, max_n, s);
+  }
 }
 
 #define OSM_MM_TYPES(X) \
