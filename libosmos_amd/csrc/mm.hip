@@ -548,30 +548,27 @@ template <uint32_t T> constexpr bool direct() {
   return T == kQ4_0 || T == kQ3_K || T == kQ4_K || T == kIQ1_S || T == kIQ1_M || T == kIQ2_XXS || T == kIQ3_XXS;
 }
 
-// F32 rows to the tiled f16: a thread 8 columns of one token (16 bytes out); rows at or past n zero. Rows: token t is
-// row idx[t] of x (-1: zero), read as two float4s
-template <bool Rows>
+// F32 rows to the tiled f16: a thread 8 columns of one token, in the order the halves lie in x16 (a 16 x 16 fragment's 32
+// threads: token by token, two a token), so a wave stores 1 KB side by side and reads 128 bytes of each of 16 rows (by
+// rows, each wave stored 32-byte pieces of 32 fragments: 7936 slots of 7168 65 -> 32 us, 231 MB). tokens at or past n
+// zero. Rows: token t is row idx[t] of x (-1: zero). Vec: rows 16-byte aligned
+template <bool Rows, bool Vec>
 __global__ __launch_bounds__(256) void x16_kernel(const float* __restrict__ x, uint32_t xs, const int32_t* __restrict__ idx,
                                                   uint32_t n, uint32_t cols, _Float16* __restrict__ x16,
                                                   int32_t* __restrict__ overflow) {
-  const uint32_t g = blockIdx.x * 256 + threadIdx.x, groups = cols / 8;
-  const uint32_t t = g / groups, c = (g % groups) * 8;
-  const uint32_t n16 = (n + kTile - 1) / kTile * kTile;
-  if (t >= n16) return;
+  const uint32_t g = blockIdx.x * 256 + threadIdx.x, frag = g / 32, per = cols / kTile;
+  const uint32_t t = frag / per * kTile + g % 32 / 2, c = frag % per * kTile + g % 2 * 8;
+  if (frag / per >= (n + kTile - 1) / kTile) return;
   const float* src = nullptr;
   if (t < n) {
-    if constexpr (Rows) {
-      const int32_t r = idx[t];
-      if (r >= 0) src = x + (uint64_t) r * xs + c;
-    } else {
-      src = x + (uint64_t) t * xs + c;
-    }
+    const int64_t r = Rows ? (int64_t) idx[t] : (int64_t) t;
+    if (r >= 0) src = x + (uint64_t) r * xs + c;
   }
   half8 h;
   bool over = false;
   if (src) {
     float v[8];
-    if constexpr (Rows) {
+    if constexpr (Vec) {
       const float4 a = ((const float4*) src)[0], b = ((const float4*) src)[1];
       v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
     } else {
@@ -584,7 +581,7 @@ __global__ __launch_bounds__(256) void x16_kernel(const float* __restrict__ x, u
 #pragma unroll
     for (int i = 0; i < 8; i++) h[i] = (_Float16) 0.0f;
   }
-  *(half8*) (x16 + x16_at(t, c, cols)) = h;
+  *(half8*) (x16 + (uint64_t) g * 8) = h;
   if (over && overflow) *overflow = 1;
 }
 
@@ -713,8 +710,11 @@ extern "C" OSM_API bool mm_x16(const float* x, uint32_t xs, uint32_t n, uint32_t
                                void* stream) {
   if (!x || !x16 || (uintptr_t) x16 % 16 || !n || n > MM_MAX_TOKENS || !cols || cols % 16 || xs < cols) return false;
   const uint64_t threads = (uint64_t) (n + 15) / 16 * 16 * (cols / 8);
-  mm::x16_kernel<false><<<(uint32_t) ((threads + 255) / 256), 256, 0, (hipStream_t) stream>>>(
-      x, xs, nullptr, n, cols, (_Float16*) x16, overflow);
+  const uint32_t grid = (uint32_t) ((threads + 255) / 256);
+  if (xs % 4 == 0 && (uintptr_t) x % 16 == 0)
+    mm::x16_kernel<false, true><<<grid, 256, 0, (hipStream_t) stream>>>(x, xs, nullptr, n, cols, (_Float16*) x16, overflow);
+  else
+    mm::x16_kernel<false, false><<<grid, 256, 0, (hipStream_t) stream>>>(x, xs, nullptr, n, cols, (_Float16*) x16, overflow);
   return hipGetLastError() == hipSuccess;
 }
 
@@ -724,7 +724,7 @@ extern "C" OSM_API bool mm_x16_rows(const float* x, uint32_t xs, const int32_t* 
       (uintptr_t) x % 16)
     return false;
   const uint64_t threads = (uint64_t) (slots + 15) / 16 * 16 * (cols / 8);
-  mm::x16_kernel<true><<<(uint32_t) ((threads + 255) / 256), 256, 0, (hipStream_t) stream>>>(
+  mm::x16_kernel<true, true><<<(uint32_t) ((threads + 255) / 256), 256, 0, (hipStream_t) stream>>>(
       x, xs, idx, slots, cols, (_Float16*) x16, overflow);
   return hipGetLastError() == hipSuccess;
 }

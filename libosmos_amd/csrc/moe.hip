@@ -284,6 +284,38 @@ __global__ __launch_bounds__(256) void moe_sum_kernel(const float* __restrict__ 
   out[i] = __fadd_rn(sum, __fmul_rn(shared[i], sigmoid(shared_logit[t])));
 }
 
+// the same with a thread 4 values and blockIdx.y the token (dim a multiple of 4, 16-aligned rows): the picks' rows loaded
+// 8 at a time before their products are added in order. HBM-bound: 512 tokens x 8 picks of 7168 (147 MB) 64 -> 24 us
+constexpr int kSumPicks = 8;
+__global__ __launch_bounds__(256) void moe_sum4_kernel(const float* __restrict__ y, const int32_t* __restrict__ where,
+                                                       const float* __restrict__ w, uint32_t k, uint32_t dim,
+                                                       const float* __restrict__ shared,
+                                                       const float* __restrict__ shared_logit, float* __restrict__ out) {
+  const uint32_t t = blockIdx.y, d = (blockIdx.x * 256 + threadIdx.x) * 4;
+  if (d >= dim) return;
+  float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (uint32_t j0 = 0; j0 < k; j0 += kSumPicks) {
+    const uint32_t n = min(k - j0, (uint32_t) kSumPicks);
+    float4 v[kSumPicks];
+    float wj[kSumPicks];
+#pragma unroll
+    for (uint32_t j = 0; j < kSumPicks; j++) {  // (past the picks: the last again, not added)
+      const uint32_t at = t * k + j0 + min(j, n - 1);
+      v[j] = *(const float4*) (y + (uint64_t) where[at] * dim + d), wj[j] = w[at];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kSumPicks; j++)
+      if (j < n) {  // (uniform)
+        s[0] = __fadd_rn(s[0], __fmul_rn(v[j].x, wj[j])), s[1] = __fadd_rn(s[1], __fmul_rn(v[j].y, wj[j]));
+        s[2] = __fadd_rn(s[2], __fmul_rn(v[j].z, wj[j])), s[3] = __fadd_rn(s[3], __fmul_rn(v[j].w, wj[j]));
+      }
+  }
+  const float g = sigmoid(shared_logit[t]);
+  const float4 h = *(const float4*) (shared + (uint64_t) t * dim + d);
+  *(float4*) (out + (uint64_t) t * dim + d) = float4{__fadd_rn(s[0], __fmul_rn(h.x, g)), __fadd_rn(s[1], __fmul_rn(h.y, g)),
+                                                     __fadd_rn(s[2], __fmul_rn(h.z, g)), __fadd_rn(s[3], __fmul_rn(h.w, g))};
+}
+
 // ---- q4x_swiglu (kernels/q4x_moe.hip:167-170): a thread 4 values, each silu(g) u (swiglu_rows_kernel's expression),
 // and, with a side output, its f16 at its (row, column) of the tiled x16 ----
 struct Side {
@@ -326,6 +358,17 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(float* __restrict__ ds
   if (i < (uint64_t) n * len) dst[i] = src[(uint64_t) idx[i / len] * len + i % len];
 }
 
+// the same with a thread 4 values and blockIdx.y a row (len a multiple of 4, 16-aligned rows; rows past the grid's most by
+// strides): 4096 rows of 7168 (117 MB written) 60 -> 35 us
+constexpr uint32_t kGridY = 65535;
+__global__ __launch_bounds__(256) void gather_rows4_kernel(float* __restrict__ dst, const float* __restrict__ src,
+                                                           const int32_t* __restrict__ idx, uint32_t n, uint32_t len) {
+  const uint32_t c = (blockIdx.x * 256 + threadIdx.x) * 4;
+  if (c >= len) return;
+  for (uint32_t r = blockIdx.y; r < n; r += gridDim.y)
+    *(float4*) (dst + (uint64_t) r * len + c) = *(const float4*) (src + (uint64_t) idx[r] * len + c);
+}
+
 // the stream held until *flag (host memory the GPU maps) holds value, with or without its top bit (the host's mark of
 // a failed job) - one thread polling it with system-scope acquire loads (vector loads: never the scalar cache, which
 // would not see the host's store), a short sleep (2 x 64 clocks) between polls. the wait is bounded by the wall clock
@@ -364,7 +407,9 @@ __global__ __launch_bounds__(256) void copy_rows_kernel(float* __restrict__ dst,
   }
 }
 
-// y[t][d] = sum over j in order of src[idx[t m + j]][d] (from 0), then add's (kernels/ops.hip:515-525); 4 values a thread
+// y[t][d] = sum over j in order of src[idx[t m + j]][d] (from 0), then add's (kernels/ops.hip:515-525); a thread a value,
+// its rows' values loaded 8 at a time before they are added (one at a time, each load waited for the index and the row
+// before it: 4 tokens x 10 rows of 2048 6.2 -> 4.5 us)
 __global__ __launch_bounds__(256) void gather_sum_kernel(float* __restrict__ y, const float* __restrict__ src,
                                                          const int32_t* __restrict__ idx, uint32_t m, uint32_t n,
                                                          uint32_t dim, const float* __restrict__ add) {
@@ -372,7 +417,16 @@ __global__ __launch_bounds__(256) void gather_sum_kernel(float* __restrict__ y, 
   if (i >= (uint64_t) n * dim) return;
   const uint32_t t = (uint32_t) (i / dim), d = (uint32_t) (i % dim);
   float s = 0.0f;
-  for (uint32_t j = 0; j < m; j++) s = __fadd_rn(s, src[(uint64_t) idx[t * m + j] * dim + d]);
+  for (uint32_t j0 = 0; j0 < m; j0 += kSumPicks) {
+    const uint32_t left = min(m - j0, (uint32_t) kSumPicks);
+    float v[kSumPicks];
+#pragma unroll
+    for (uint32_t j = 0; j < kSumPicks; j++)  // (past the rows: the last again, not added)
+      v[j] = src[(uint64_t) idx[t * m + j0 + min(j, left - 1)] * dim + d];
+#pragma unroll
+    for (uint32_t j = 0; j < kSumPicks; j++)
+      if (j < left) s = __fadd_rn(s, v[j]);
+  }
   y[i] = add ? __fadd_rn(s, add[i]) : s;
 }
 
@@ -383,6 +437,10 @@ struct LaneBases {
   uint64_t bytes[3];
 };
 
+// one workgroup. every pass reads LDS: the ids are copied there first, an expert's rows and entries are one packed
+// prefix sum over the experts (a wave's shifts, then the 16 waves' totals), and a pick ranks itself among its token's
+// picks instead of a thread sorting them. It is latency (a dozen barriers and short loops): 40 picks of 512 experts
+// 16.6 -> 4.5 us, where the scan's 20 barriers, the ranks' global loads and the sort's scratch array were most of it
 __global__ __launch_bounds__(kLaneThreads) void lane_tables_kernel(const int32_t* __restrict__ ids, uint32_t n_tok,
                                                                    uint32_t k, uint32_t n_exp, LaneBases b,
                                                                    int32_t* __restrict__ tok, int32_t* __restrict__ pair,
@@ -391,78 +449,106 @@ __global__ __launch_bounds__(kLaneThreads) void lane_tables_kernel(const int32_t
                                                                    const void** __restrict__ wu,
                                                                    const void** __restrict__ wd,
                                                                    int32_t* __restrict__ order) {
-  __shared__ int count[kMaxExperts], start[kMaxExperts], estart[kMaxExperts];
+  constexpr int kWaves = kLaneThreads / kWave;
+  __shared__ int count[kMaxExperts], start[kMaxExperts], wsum[kWaves];
+  __shared__ __attribute__((aligned(16))) int id[OSMOS_LANE_MAX_PAIRS];
   __shared__ int row_of[OSMOS_LANE_MAX_PAIRS];
-  __shared__ int n_entries;
   const uint32_t n = n_tok * k, e = threadIdx.x;
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   count[e] = 0;
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < n; i += kLaneThreads) atomicAdd(&count[ids[i]], 1);
-  __syncthreads();
-  const int c = e < n_exp ? count[e] : 0, ne = (c + MV_MAX_TOKENS - 1) / MV_MAX_TOKENS;
-  start[e] = c, estart[e] = ne;
-  __syncthreads();
-  for (uint32_t d = 1; d < kMaxExperts; d <<= 1) {  // inclusive scans, then each less its own
-    const int a = e >= d ? start[e - d] : 0, bb = e >= d ? estart[e - d] : 0;
-    __syncthreads();
-    start[e] += a, estart[e] += bb;
-    __syncthreads();
+  for (uint32_t i = threadIdx.x; i < n; i += kLaneThreads) {
+    const int v = ids[i];
+    id[i] = v;
+    atomicAdd(&count[v], 1);
   }
-  if (e == kMaxExperts - 1) n_entries = estart[e];
-  start[e] -= c, estart[e] -= ne;
+  __syncthreads();
+  // rows in the low half, entries (of at most MV_MAX_TOKENS rows) in the high: both sums at most 4096
+  const int c = e < n_exp ? count[e] : 0, ne = (c + MV_MAX_TOKENS - 1) / MV_MAX_TOKENS;
+  int v = c | ne << 16;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int u = __shfl_up(v, o, kWave);
+    if (lane >= o) v += u;
+  }
+  if (lane == kWave - 1) wsum[wave] = v;
+  __syncthreads();
+  int before = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < kWaves; w++) {
+    const int u = wsum[w];
+    before += w < wave ? u : 0, total += u;
+  }
+  v += before - (c | ne << 16);
+  const int row0 = v & 0xFFFF, entry0 = v >> 16;
+  start[e] = row0;
   __syncthreads();
   // each pick's row: its expert's first plus the expert's picks before it (sorted by expert, then pick)
   for (uint32_t i = threadIdx.x; i < n; i += kLaneThreads) {
-    const int32_t ex = ids[i];
+    const int ex = id[i];
     int rank = 0;
-    for (uint32_t j = 0; j < i; j++) rank += ids[j] == ex;
+    uint32_t j = 0;
+    for (; j + 4 <= i; j += 4) {
+      const int4 q = *(const int4*) (id + j);
+      rank += (q.x == ex) + (q.y == ex) + (q.z == ex) + (q.w == ex);
+    }
+    for (; j < i; j++) rank += id[j] == ex;
     const int r = start[ex] + rank;
     row_of[i] = r, tok[r] = (int32_t) (i / k), pair[r] = (int32_t) i;
   }
-  // each expert's entries of at most MV_MAX_TOKENS rows, in order
-  if (c)
-    for (int p = 0; p < ne; p++) {
-      const int en = estart[e] + p;
-      cnt[en] = c - p * MV_MAX_TOKENS < MV_MAX_TOKENS ? c - p * MV_MAX_TOKENS : MV_MAX_TOKENS;
-      xrow[en] = start[e] + p * MV_MAX_TOKENS;
-      wg[en] = b.base[0] + (uint64_t) e * b.bytes[0];
-      wu[en] = b.base[1] + (uint64_t) e * b.bytes[1];
-      wd[en] = b.base[2] + (uint64_t) e * b.bytes[2];
-    }
+  // each expert's entries, in order
+  for (int p = 0; p < ne; p++) {
+    const int en = entry0 + p;
+    cnt[en] = min(c - p * MV_MAX_TOKENS, MV_MAX_TOKENS);
+    xrow[en] = row0 + p * MV_MAX_TOKENS;
+    wg[en] = b.base[0] + (uint64_t) e * b.bytes[0];
+    wu[en] = b.base[1] + (uint64_t) e * b.bytes[1];
+    wd[en] = b.base[2] + (uint64_t) e * b.bytes[2];
+  }
+  for (uint32_t en = (uint32_t) (total >> 16) + threadIdx.x; en < n; en += kLaneThreads) cnt[en] = 0, xrow[en] = 0;
   __syncthreads();
-  for (uint32_t en = (uint32_t) n_entries + threadIdx.x; en < n; en += kLaneThreads) cnt[en] = 0, xrow[en] = 0;
-  // a token's rows in ascending order (its experts ascending: rows ascend by expert)
-  for (uint32_t t = threadIdx.x; t < n_tok; t += kLaneThreads) {
-    int r[kMaxK];
-    for (uint32_t j = 0; j < k; j++) {
-      int v = row_of[t * k + j], q = (int) j;
-      while (q > 0 && r[q - 1] > v) r[q] = r[q - 1], q--;
-      r[q] = v;
-    }
-    for (uint32_t j = 0; j < k; j++) order[t * k + j] = r[j];
+  // a token's rows in ascending order (its experts ascending: rows ascend by expert): each pick's place among them
+  for (uint32_t i = threadIdx.x; i < n; i += kLaneThreads) {
+    const uint32_t t0 = i / k * k;
+    const int r = row_of[i];
+    int place = 0;
+    for (uint32_t j = t0; j < t0 + k; j++) place += row_of[j] < r;
+    order[t0 + place] = r;
   }
 }
 
 inline unsigned grid256(uint64_t n) { return (unsigned) ((n + 255) / 256); }
+inline bool aligned16(const void* a, const void* b, const void* c) { return (((uintptr_t) a | (uintptr_t) b | (uintptr_t) c) & 15) == 0; }
 
-// ---- q4x_swiglu_rows (kernels/q4x_moe.hip:235-253): a thread 8 columns of a slot, silu(g) u (swiglu_kernel's
-// expression) rounded to f16 as mm_x16_rows rounds ----
+// ---- q4x_swiglu_rows (kernels/q4x_moe.hip:235-253): a thread 8 columns of a slot in x16's own order (mm.hip's x16_kernel),
+// silu(g) u (swiglu_kernel's expression) rounded to f16 as mm_x16_rows rounds. Vec: g and u 16-byte aligned (7936 slots
+// of 2048, 99 MB: 69 -> 22 us) ----
+template <bool Vec>
 __global__ __launch_bounds__(256) void swiglu_rows_kernel(const float* __restrict__ g, const float* __restrict__ u,
                                                           uint32_t ff, const int32_t* __restrict__ idx, uint32_t slots,
                                                           _Float16* __restrict__ x16, int32_t* __restrict__ overflow) {
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x, groups = ff / 8;
-  const uint32_t sl = i / groups, c = (i % groups) * 8;
+  const uint64_t i = (uint64_t) blockIdx.x * 256 + threadIdx.x;
+  const uint32_t frag = (uint32_t) (i / 32), per = ff / kX16Tile;
+  const uint32_t sl = frag / per * kX16Tile + (uint32_t) (i % 32) / 2, c = frag % per * kX16Tile + (uint32_t) (i % 2) * 8;
   if (sl >= slots) return;
   const int32_t r = idx[sl];
   typedef _Float16 half8 __attribute__((ext_vector_type(8)));
   half8 h;
   bool over = false;
+  float gv[8], uv[8];
+  const uint64_t at = (uint64_t) (r >= 0 ? r : 0) * ff + c;
+  if constexpr (Vec) {
+    const float4 a = ((const float4*) (g + at))[0], b = ((const float4*) (g + at))[1];
+    const float4 e = ((const float4*) (u + at))[0], f = ((const float4*) (u + at))[1];
+    gv[0] = a.x, gv[1] = a.y, gv[2] = a.z, gv[3] = a.w, gv[4] = b.x, gv[5] = b.y, gv[6] = b.z, gv[7] = b.w;
+    uv[0] = e.x, uv[1] = e.y, uv[2] = e.z, uv[3] = e.w, uv[4] = f.x, uv[5] = f.y, uv[6] = f.z, uv[7] = f.w;
+  } else {
 #pragma unroll
-  for (int j = 0; j < 8; j++) {
-    const uint64_t at = (uint64_t) (r >= 0 ? r : 0) * ff + c + j;
-    h[j] = x16_round(r >= 0 ? __fmul_rn(silu(g[at]), u[at]) : 0.0f, over);
+    for (int j = 0; j < 8; j++) gv[j] = g[at + j], uv[j] = u[at + j];
   }
-  *(half8*) (x16 + x16_at(sl, c, ff)) = h;
+#pragma unroll
+  for (int j = 0; j < 8; j++) h[j] = x16_round(r >= 0 ? __fmul_rn(silu(gv[j]), uv[j]) : 0.0f, over);
+  *(half8*) (x16 + i * 8) = h;
   if (over) *overflow = 1;
 }
 
@@ -526,9 +612,12 @@ extern "C" OSM_API bool q4x_spin(uint32_t us, void* stream) {
 extern "C" OSM_API bool q4x_swiglu_rows(const float* g, const float* u, uint32_t ff, const int32_t* idx,
                                         uint32_t slots, void* x16, int32_t* overflow, void* stream) {
   if (!g || !u || !idx || !x16 || (uintptr_t) x16 % 16 || !overflow || !slots || !ff || ff % kX16Tile) return false;
-  const uint64_t threads = (uint64_t) slots * (ff / 8);
-  moe::swiglu_rows_kernel<<<(uint32_t) ((threads + 255) / 256), 256, 0, (hipStream_t) stream>>>(
-      g, u, ff, idx, slots, (_Float16*) x16, overflow);
+  const uint64_t threads = (uint64_t) (slots + moe::kTile - 1) / moe::kTile * moe::kTile * (ff / 8);
+  const uint32_t grid = (uint32_t) ((threads + 255) / 256);
+  if (moe::aligned16(g, u, nullptr))
+    moe::swiglu_rows_kernel<true><<<grid, 256, 0, (hipStream_t) stream>>>(g, u, ff, idx, slots, (_Float16*) x16, overflow);
+  else
+    moe::swiglu_rows_kernel<false><<<grid, 256, 0, (hipStream_t) stream>>>(g, u, ff, idx, slots, (_Float16*) x16, overflow);
   return hipGetLastError() == hipSuccess;
 }
 
@@ -536,6 +625,11 @@ extern "C" OSM_API bool q4x_moe_sum(const float* y, const int32_t* where, const 
                                     uint32_t dim, const float* shared, const float* shared_logit, float* out,
                                     void* stream) {
   if (!y || !where || !w || !shared || !shared_logit || !out || !n_tok || !k || !dim) return false;
+  if (dim % 4 == 0 && n_tok <= moe::kGridY && moe::aligned16(y, shared, out)) {
+    moe::moe_sum4_kernel<<<dim3((dim + 1023) / 1024, n_tok), 256, 0, (hipStream_t) stream>>>(y, where, w, k, dim, shared,
+                                                                                            shared_logit, out);
+    return hipGetLastError() == hipSuccess;
+  }
   moe::moe_sum_kernel<<<moe::grid256((uint64_t) n_tok * dim), 256, 0, (hipStream_t) stream>>>(y, where, w, n_tok, k, dim,
                                                                                              shared, shared_logit, out);
   return hipGetLastError() == hipSuccess;
@@ -552,6 +646,11 @@ extern "C" OSM_API bool ops_swiglu_lane(const float* g, const float* u, uint32_t
 extern "C" OSM_API bool ops_gather_rows(float* dst, const float* src, const int32_t* idx, uint32_t n, uint32_t len,
                                         void* stream) {
   if (!dst || !src || !idx || !n || !len) return false;
+  if (len % 4 == 0 && moe::aligned16(dst, src, nullptr)) {
+    moe::gather_rows4_kernel<<<dim3((len + 1023) / 1024, n < moe::kGridY ? n : moe::kGridY), 256, 0, (hipStream_t) stream>>>(
+        dst, src, idx, n, len);
+    return hipGetLastError() == hipSuccess;
+  }
   moe::gather_rows_kernel<<<moe::grid256((uint64_t) n * len), 256, 0, (hipStream_t) stream>>>(dst, src, idx, n, len);
   return hipGetLastError() == hipSuccess;
 }
