@@ -251,8 +251,9 @@ __global__ __launch_bounds__(NTH) void wide_kernel(const uint8_t* const* __restr
   uint32_t W[36];
   if constexpr (CB % 16) {
     const uintptr_t a0 = (uintptr_t) w[m] & ~(uintptr_t) 15, at = (uintptr_t) src;
+    // (the range in whole words: a word that ends past it reads as zero, and a 2-aligned matrix ends inside its last word)
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-        (void*) a0, (short) 0, (int) ((uintptr_t) w[m] - a0 + (uint64_t) rows * rb), 0x00020000);
+        (void*) a0, (short) 0, (int) (((uintptr_t) w[m] - a0 + (uint64_t) rows * rb + 3) & ~(uint64_t) 3), 0x00020000);
     const uint32_t o = (uint32_t) ((at & ~(uintptr_t) 15) - a0), sh = (uint32_t) (at & 15);
     uint32_t V[32];
 #pragma unroll
