@@ -595,6 +595,7 @@ struct G1Tab {
   const float *d, *scale;
   float* h;
   uint32_t hs;
+  int32_t most;  // (tab_kernel: a matrix's tokens at most)
 };
 
 // one gate/up tile of one token: the layer's (pick m's expert ids[m], its rows at gate + id gate_bytes, router weight
@@ -975,6 +976,157 @@ __global__ __launch_bounds__(kWave * W) void gub_kernel(GuArgs a) {
   for (; c0 < cnt; c0++) {
     __syncthreads();
     gub_pass<T, L, 1, P, W>(a, toks, c0, 1, 0, q, d, grid, wr, r0);
+  }
+}
+
+// ---- the same tiles over q8_gate_up's and q8_group_tok's pointer tables, for entries of several tokens ----
+// what they replace decoded each block from global memory in two-byte loads, a row a lane group; here a workgroup's rows
+// are staged with 16-byte loads, the codebook and the entry's x rows (NB tokens a pass) beside them, and each decoded
+// block serves the pass's tokens. decode and the loads' latency bound it. entry m: rows xrow[m] .. of cnt[m] tokens, their
+// inputs xin[row] (or row). the engine's whole sequence, 4 tokens (us): 512-expert layer of 2048 / 512, IQ3_XXS 67 -> 51;
+// 257-expert layer of 7168 / 2048, IQ1_S 304 -> 165, IQ1_M 356 -> 186, IQ2_XXS 312 -> 238, IQ3_XXS 490 -> 400
+
+// 16-byte word i of a matrix's rows (two-byte loads where it is not 16-aligned)
+__device__ __forceinline__ u32x4 tab_word(const uint8_t* p, uint32_t i, bool aligned) {
+  if (aligned) return wload((const u32x4*) p + i);
+  p += 16 * i;
+  u32x4 v;
+  v.x = osm::ld16(p) | osm::ld16(p + 2) << 16, v.y = osm::ld16(p + 4) | osm::ld16(p + 6) << 16;
+  v.z = osm::ld16(p + 8) | osm::ld16(p + 10) << 16, v.w = osm::ld16(p + 12) | osm::ld16(p + 14) << 16;
+  return v;
+}
+
+// MATS: 2 (q8_gate_up: a wave a row, its gate row in lanes 0 .. 31 and its up row in 32 .. 63) or 1 (q8_group_tok: a row
+// L lanes). R: the workgroup's rows of a matrix
+template <uint32_t T, int L, int NB, int W, int MATS>
+struct TabLds {
+  static constexpr uint32_t D = G1Max<L>::dim, R = MATS == 2 ? W : W * (kWave / L);
+  static constexpr uint32_t grid = 0, q = align16(grid_bytes<T>()), d = q + NB * D, w = d + NB * (D / 32) * 4;
+  static constexpr uint32_t total = w + align16(MATS * R * (uint32_t) row_bytes<T>(D));
+};
+
+template <uint32_t T, int S, int L, int NB, int W, int MATS>
+__global__ __launch_bounds__(kWave * W) void tab_kernel(GuArgs a, G1Tab tb) {
+  using LD = TabLds<T, L, NB, W, MATS>;
+  __shared__ __attribute__((aligned(16))) uint8_t smem[LD::total];
+  constexpr int kThreads = kWave * W;
+  constexpr uint32_t R = LD::R, per = Block<T>::values / 32, bb = Block<T>::bytes;
+  const uint32_t m = blockIdx.y, r0 = blockIdx.x * R;
+  const int cnt = min(tb.cnt[m], tb.most);
+  if (cnt <= 0) return;  // (uniform)
+  const uint32_t rb = (uint32_t) row_bytes<T>(a.dim), nblk = a.dim / 32, per_seg = R * rb / 16, out0 = (uint32_t) tb.xrow[m];
+  GridStage<T, kThreads> gs;
+  grid_load(gs);
+  __builtin_amdgcn_sched_barrier(0);
+  u32x4 wv[MATS * S];
+#pragma unroll
+  for (int mt = 0; mt < MATS; mt++) {
+    const uint8_t* src = table_at(mt ? tb.wu : tb.wg, m) + (uint64_t) r0 * rb;
+    const bool aligned = ((uintptr_t) src & 15) == 0;
+#pragma unroll
+    for (uint32_t u = 0; u < (uint32_t) S; u++) wv[mt * S + u] = tab_word(src, min(u * kThreads + threadIdx.x, per_seg - 1), aligned);
+  }
+  int8_t* q = (int8_t*) (smem + LD::q);
+  float* d = (float*) (smem + LD::d);
+  // the x rows of tokens c0 .. c0 + nb - 1 of the entry
+  auto xcopy = [&](int c0, int nb) __attribute__((always_inline)) {
+    const uint32_t wpr = a.dim / 16;
+    auto row = [&](uint32_t b) __attribute__((always_inline)) {
+      const uint32_t r = out0 + c0 + b;
+      return (uint64_t) (tb.xin ? (uint32_t) tb.xin[r] : r);
+    };
+    for (uint32_t i = threadIdx.x; i < nb * wpr; i += kThreads)
+      ((u32x4*) q)[i] = ((const u32x4*) (tb.q + row(i / wpr) * a.dim))[i % wpr];
+    for (uint32_t i = threadIdx.x; i < nb * nblk; i += kThreads) d[i] = tb.d[row(i / nblk) * nblk + i % nblk];
+  };
+  int c0 = 0, nb = cnt >= NB ? NB : 1;
+  xcopy(0, nb);
+  grid_store(gs, smem + LD::grid);
+#pragma unroll
+  for (int mt = 0; mt < MATS; mt++)
+#pragma unroll
+    for (uint32_t u = 0; u < (uint32_t) S; u++) {
+      const uint32_t l = u * kThreads + threadIdx.x;
+      if (l < per_seg) ((u32x4*) (smem + LD::w))[mt * per_seg + l] = wv[mt * S + u];
+    }
+  __syncthreads();
+  const auto* grid = (const typename GridOf<T>::E*) (smem + LD::grid);
+  const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, ll = lane % L;
+  // q8_gate_up at 16 lanes: a half-wave a row, each chain split between lanes ll and ll + 16 as in gub_pass
+  constexpr bool kHalves = MATS == 2 && L == 16;
+  const uint32_t row = MATS == 2 ? wave : wave * (kWave / L) + lane / L;
+  const uint8_t* wr = smem + LD::w + (MATS == 2 ? (lane / 32) * R + row : row) * rb;
+  auto pass = [&](auto nbc) __attribute__((always_inline)) {
+    constexpr int N = decltype(nbc)::value;
+    float v[N];
+    if constexpr (kHalves) {
+      const uint32_t half = lane / 16 % 2, C = nblk / 16, CA = (C + 1) / 2, i0 = half ? CA : 0, n_i = half ? C - CA : CA;
+      float sub[2][N], xd[2][N];
+#pragma unroll
+      for (uint32_t k = 0; k < 2; k++) {
+#pragma unroll
+        for (int b = 0; b < N; b++) sub[k][b] = 0.0f, xd[k][b] = 0.0f;
+        if (k < n_i) {
+          const uint32_t sb = ll + 16 * (i0 + k);
+          Codes c;
+          codes<T>((lbytes) (wr + (sb / per) * bb), (int) (sb % per), c, grid);
+#pragma unroll
+          for (int b = 0; b < N; b++) {
+            int x[8];
+            load_x(q, (b * nblk + sb) * 32, x);
+            sub[k][b] = block_sum<T>(c, x), xd[k][b] = d[b * nblk + sb];
+          }
+        }
+      }
+#pragma unroll
+      for (int b = 0; b < N; b++) {
+        float acc = 0.0f;
+#pragma unroll
+        for (uint32_t k = 0; k < 2; k++)
+          if (k < CA) acc = __builtin_fmaf(xd[k][b], sub[k][b], acc);
+        acc = xor_lane(acc, 16);
+#pragma unroll
+        for (uint32_t k = 0; k < 2; k++)
+          if (k < C - CA) acc = __builtin_fmaf(xd[k][b], sub[k][b], acc);
+        v[b] = tree<16>(acc);
+      }
+    } else {
+#pragma unroll
+      for (int b = 0; b < N; b++) v[b] = 0.0f;
+      for (uint32_t sb = ll; sb < nblk; sb += L) {
+        Codes c;
+        codes<T>((lbytes) (wr + (sb / per) * bb), (int) (sb % per), c, grid);
+#pragma unroll
+        for (int b = 0; b < N; b++) {
+          int x[8];
+          load_x(q, (b * nblk + sb) * 32, x);
+          v[b] = __builtin_fmaf(d[b * nblk + sb], block_sum<T>(c, x), v[b]);
+        }
+      }
+#pragma unroll
+      for (int b = 0; b < N; b++) v[b] = tree<L>(v[b]);
+    }
+#pragma unroll
+    for (int b = 0; b < N; b++) {
+      const uint32_t out = out0 + c0 + b;
+      if constexpr (MATS == 2) {
+        const float g = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[b]), 16));
+        const float u = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[b]), 48));
+        if (lane == 0) tb.h[(uint64_t) out * tb.hs + r0 + row] = lane_swiglu(g, u, a.lim, tb.scale[tb.win ? (uint32_t) tb.win[out] : out]);
+      } else {
+        if (ll == 0) tb.h[(uint64_t) out * tb.hs + r0 + row] = v[b];
+      }
+    }
+  };
+  for (;;) {  // NB tokens a pass while that many are left, then one a pass
+    if (nb == NB) pass(std::integral_constant<int, NB>{});
+    else pass(std::integral_constant<int, 1>{});
+    c0 += nb;
+    if (c0 >= cnt) break;
+    nb = cnt - c0 >= NB ? NB : 1;
+    __syncthreads();  // (the pass's codes read)
+    xcopy(c0, nb);
+    __syncthreads();
   }
 }
 

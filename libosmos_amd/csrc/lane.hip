@@ -579,7 +579,7 @@ bool tab_launch_l(const Args& a, hipStream_t s, uint32_t words) {
   fused::GuArgs ga{};
   ga.dim = a.cols, ga.ff = a.rows, ga.lim = a.lim;
   const fused::G1Tab tb = {(const uint8_t* const*) a.wg, (const uint8_t* const*) a.wu, a.cnt, a.xrow, a.xin, a.win,
-                           a.q, a.d, a.scale, a.y, a.ys};
+                           a.q, a.d, a.scale, a.y, a.ys, 1};
   const dim3 grid(a.rows / fused::kG1Rows, a.n);
   constexpr int kT = fused::kG1Threads;
   if (words <= (uint32_t) kT) fused::gu1_tab_kernel<T, 1, L><<<grid, kT, 0, s>>>(ga, tb);
@@ -595,6 +595,36 @@ bool tab_launch(const Args& a, hipStream_t s, bool* taken) {
   if (*taken && a.cols % 1024 == 0 && a.cols >= 4096 && a.cols <= fused::G1Max<32>::dim)
     return tab_launch_l<T, 32>(a, s, words);
   *taken = false;
+  return false;
+}
+
+// several tokens an entry on the staged tiles (fused::tab_kernel): q8_gate_up (MATS 2) where tab_launch's shapes hold,
+// q8_group_tok (MATS 1) over whole workgroups of rows (false in *taken: not taken)
+template <uint32_t T, int L, int MATS>
+bool tabs_launch_l(const Args& a, int most, hipStream_t s, bool* taken) {
+  constexpr int NB = L == 16 ? 4 : 2, W = L == 16 || fused::grid_bytes<T>() >= 8192 ? 8 : 4, kT = kWave * W;
+  using LD = fused::TabLds<T, L, NB, W, MATS>;
+  const uint32_t rb = (uint32_t) row_bytes<T>(a.cols), words = LD::R * rb / 16;
+  *taken = LD::total <= 64 * 1024 && a.rows % LD::R == 0 && (LD::R * rb) % 16 == 0 &&
+           words <= (uint32_t) fused::kG1Slots * kT && ((uintptr_t) a.q & 15) == 0;
+  if (!*taken) return false;
+  if constexpr (LD::total <= 64 * 1024) {
+    fused::GuArgs ga{};
+    ga.dim = a.cols, ga.ff = a.rows, ga.lim = a.lim;
+    const fused::G1Tab tb = {(const uint8_t* const*) a.wg, (const uint8_t* const*) a.wu, a.cnt, a.xrow, a.xin, a.win,
+                             a.q, a.d, a.scale, a.y, a.ys, most};
+    const dim3 grid(a.rows / LD::R, a.n);
+    if (words <= (uint32_t) kT) fused::tab_kernel<T, 1, L, NB, W, MATS><<<grid, kT, 0, s>>>(ga, tb);
+    else if (words <= 2u * kT) fused::tab_kernel<T, 2, L, NB, W, MATS><<<grid, kT, 0, s>>>(ga, tb);
+    else fused::tab_kernel<T, fused::kG1Slots, L, NB, W, MATS><<<grid, kT, 0, s>>>(ga, tb);
+  }
+  return hipGetLastError() == hipSuccess;
+}
+template <uint32_t T, int MATS>
+bool tabs_launch(const Args& a, int most, hipStream_t s, bool* taken) {
+  *taken = false;
+  if (a.cols % 512 == 0 && a.cols <= fused::G1Max<16>::dim) return tabs_launch_l<T, 16, MATS>(a, most, s, taken);
+  if (a.cols % 1024 == 0 && a.cols >= 4096 && a.cols <= fused::G1Max<32>::dim) return tabs_launch_l<T, 32, MATS>(a, most, s, taken);
   return false;
 }
 
@@ -622,6 +652,16 @@ bool by_lanes(const Args& a, bool fused, hipStream_t s, uint32_t tiles = 1) {
 template <uint32_t T>
 bool by_tokens(const Args& a, uint32_t max_cnt, bool fused, hipStream_t s) {
   if (a.cols % Block<T>::values) return false;
+  // several tokens an entry, or one where the tile beats the per-row kernels (us a layer of 9 or 10 experts: 2048 -> 7168
+  // IQ3_XXS 93.9 -> 68.4, IQ1_S 61.5 -> 54.8, IQ1_M 66.0 -> 60.6, IQ2_XXS 74.2 -> 71.8; 512 -> 2048 IQ3_XXS 25.4 -> 24.9, the
+  // others slower). one matrix alone keeps the kernels above: they put more waves on it
+  constexpr bool kIq = T != kQ2_K && T != kQ4_0 && T != kQ4_K && T != kQ3_K;
+  if (a.n > 1 && (max_cnt > 1 || (!fused && kIq && (a.cols >= 1024 || T == kIQ3_XXS)))) {
+    bool taken = false;
+    const int most = max_cnt > 4 ? 8 : (int) max_cnt;  // (as the token tiles below)
+    const bool ok = fused ? tabs_launch<T, 2>(a, most, s, &taken) : tabs_launch<T, 1>(a, most, s, &taken);
+    if (taken) return ok;
+  }
   switch (max_cnt) {
     case 1: return by_lanes<T, 1>(a, fused, s);
     case 2: return by_lanes<T, 2>(a, fused, s);
