@@ -200,7 +200,7 @@ __global__ __launch_bounds__(W * kWave) void kernel(Args a) {
       const uint8_t* base = w + (uint64_t) r * kRb;
 #pragma unroll
       for (uint32_t u = 0; u < kPer; u++) {
-        const uint32_t o = (u * kThreads + threadIdx.x) % kWr * WB;
+        const uint32_t o = min(u * kThreads + threadIdx.x, kWords - 1) % kWr * WB;  // (woff's word)
         wr[u] = gload<word>(base + woff[u] - (o < lim ? 0 : o - (lim - WB)));  // (past a short round: its last word)
       }
     }
