@@ -983,7 +983,9 @@ __global__ __launch_bounds__(kWave * W) void gub_kernel(GuArgs a) {
 // what they replace decoded each block from global memory in two-byte loads, a row a lane group; here a workgroup's rows
 // are staged with 16-byte loads, the codebook and the entry's x rows (NB tokens a pass) beside them, and each decoded
 // block serves the pass's tokens. decode and the loads' latency bound it. entry m: rows xrow[m] .. of cnt[m] tokens, their
-// inputs xin[row] (or row). the engine's whole sequence, 4 tokens (us): 512-expert layer of 2048 / 512, IQ3_XXS 67 -> 51;
+// inputs xin[row] (or row). which calls come here, with both sides' times: lane.hip's tabs_pay. what is left of a count
+// after passes of NB goes in one pass of its size (as passes of one token, 4 of gate/up 512 x 2048 with 3 tokens each took,
+// us: IQ3_XXS 6.4, IQ2_XXS 6.0; in one 4.9, 4.2). the engine's whole sequence, 4 tokens (us): 512-expert layer of 2048 / 512, IQ3_XXS 67 -> 51;
 // 257-expert layer of 7168 / 2048, IQ1_S 304 -> 165, IQ1_M 356 -> 186, IQ2_XXS 312 -> 238, IQ3_XXS 490 -> 400
 
 // 16-byte word i of a matrix's rows (two-byte loads where it is not 16-aligned)
@@ -1007,6 +1009,7 @@ struct TabLds {
 
 template <uint32_t T, int S, int L, int NB, int W, int MATS>
 __global__ __launch_bounds__(kWave * W) void tab_kernel(GuArgs a, G1Tab tb) {
+  static_assert(NB == 2 || NB == 4, "passes of 1 to NB tokens");
   using LD = TabLds<T, L, NB, W, MATS>;
   __shared__ __attribute__((aligned(16))) uint8_t smem[LD::total];
   constexpr int kThreads = kWave * W;
@@ -1039,7 +1042,7 @@ __global__ __launch_bounds__(kWave * W) void tab_kernel(GuArgs a, G1Tab tb) {
       ((u32x4*) q)[i] = ((const u32x4*) (tb.q + row(i / wpr) * a.dim))[i % wpr];
     for (uint32_t i = threadIdx.x; i < nb * nblk; i += kThreads) d[i] = tb.d[row(i / nblk) * nblk + i % nblk];
   };
-  int c0 = 0, nb = cnt >= NB ? NB : 1;
+  int c0 = 0, nb = min(cnt, NB);
   xcopy(0, nb);
   grid_store(gs, smem + LD::grid);
 #pragma unroll
@@ -1118,12 +1121,14 @@ __global__ __launch_bounds__(kWave * W) void tab_kernel(GuArgs a, G1Tab tb) {
       }
     }
   };
-  for (;;) {  // NB tokens a pass while that many are left, then one a pass
+  for (;;) {  // NB tokens a pass while that many are left, then the rest in one: each block decoded once a pass
     if (nb == NB) pass(std::integral_constant<int, NB>{});
-    else pass(std::integral_constant<int, 1>{});
+    else if (nb == 1) pass(std::integral_constant<int, 1>{});
+    else if (nb == NB / 2) pass(std::integral_constant<int, NB / 2>{});
+    else if constexpr (NB == 4) pass(std::integral_constant<int, 3>{});
     c0 += nb;
     if (c0 >= cnt) break;
-    nb = cnt - c0 >= NB ? NB : 1;
+    nb = min(cnt - c0, NB);
     __syncthreads();  // (the pass's codes read)
     xcopy(c0, nb);
     __syncthreads();

@@ -598,33 +598,71 @@ bool tab_launch(const Args& a, hipStream_t s, bool* taken) {
   return false;
 }
 
-// several tokens an entry on the staged tiles (fused::tab_kernel): q8_gate_up (MATS 2) where tab_launch's shapes hold,
+// which calls over pointer tables the staged tiles (fused::tab_kernel) serve: n entries of at most max_cnt tokens, their
+// counts known to the device alone. routed: what a decode step's routing makes (an entry a pick, so n = tokens x k, most of
+// one token), and not a table of full entries, where the per-row kernels decode a block as often and put more waves on it.
+// measured (us, per-row kernels -> tiles, weights from HBM; 4 tokens x 10 of 512 experts): gate/up 512 x 2048 IQ3_XXS 33.7 ->
+// 18.7, Q4_K 25.0 -> 16.9, IQ1_M 24.9 -> 18.1, IQ2_XXS 22.4 -> 19.7, Q3_K 26.2 -> 27.2 (2 tokens 18.6 -> 15.8); 2048 x 7168
+// IQ1_S 229 -> 105, IQ2_XXS 238 -> 162, IQ2_XS 232 -> 184, Q4_0 201 -> 178 (but 1536 x 4096 90.8 -> 95.6); 768 x 1024 IQ3_XXS
+// 26.8 -> 22.2, IQ2_XXS 18.9 -> 22.8; q8_group_tok 2048 x 512 IQ3_XXS 17.5 -> 14.7, Q4_K 20.0 -> 12.3, IQ1_M 16.2 -> 14.4,
+// IQ2_XXS 13.4 -> 14.5; 1024 x 1024 IQ2_XXS 13.4 -> 11.2; 2048 x 7168 IQ1_S 142 -> 51. full entries of 8 tokens: 8 of gate/up
+// 2048 x 7168 IQ2_XXS 97 -> 138, 8 of 512 x 2048 IQ1_S 11.0 -> 13.7, 64 of it 57 -> 83; few workgroups: q8_group_tok, 2 of
+// 2048 x 512 at 2 tokens, IQ1_S 2.8 -> 3.6. one token, 10 of 2048 x 2048: IQ3_XXS 17.2 -> 10.8, IQ1_S 9.1 -> 8.1, IQ2_XS 10.5 ->
+// 11.3 (9 of 7168 x 2048 26.5 -> 24.5); of 1024 x 1024 IQ1_M 4.5 -> 4.9
+template <uint32_t T, int L, int MATS>
+constexpr bool tabs_serve() { return T != kQ3_K ? !(T == kQ4_0 && MATS == 2 && L == 32) : MATS == 2 && L == 16; }
+template <uint32_t T, int L, int MATS>
+bool tabs_pay(uint32_t n, uint32_t max_cnt, uint32_t rows, uint32_t cols, uint32_t wgs) {
+  constexpr bool kIq1 = T == kIQ1_S || T == kIQ1_M, kIq = T != kQ2_K && T != kQ4_0 && T != kQ4_K && T != kQ3_K;
+  const bool routed = n >= 4 * max_cnt, some = n >= 2 * max_cnt, few = max_cnt <= 4, one_step = n <= 16 * max_cnt;
+  constexpr uint32_t kOne = T == kIQ3_XXS ? 128 : T == kIQ2_XXS || T == kIQ2_XS ? 1024 : 192;
+  if (max_cnt == 1) return MATS == 1 && kIq && (L == 32 || (wgs >= kOne && (T == kIQ3_XXS || cols > 1024)));
+  if constexpr (MATS == 2 && L == 16) {
+    if constexpr (T == kQ3_K) return cols > 1536 && (max_cnt <= 3 || (few && wgs <= 256));
+    if constexpr (T == kIQ3_XXS || T == kQ4_K)
+      return cols > (T == kQ4_K ? 1536 : 1024) || (cols >= 1024 && (few || some) && one_step);
+    return cols > (T == kQ2_K || T == kQ4_0 ? 1024 : 1536) && (few || routed) && (one_step || T == kIQ1_M || (T == kQ2_K && cols > 1536));
+  }
+  if constexpr (MATS == 2) {
+    if constexpr (kIq1) return max_cnt <= 3 || some;
+    return max_cnt == 2 || (routed && (one_step || T == kIQ2_XXS || T == kQ2_K));
+  }
+  if constexpr (L == 32) return kIq1 ? max_cnt <= 3 || wgs >= 512 : max_cnt == 2 || (T == kIQ2_XS ? routed : some);
+  if constexpr (T == kIQ3_XXS) return cols > 1024 || wgs >= 256;
+  if (wgs < 192) return false;
+  if (cols < 1024) return T == kQ4_K || ((T == kIQ1_M || T == kQ2_K) && max_cnt >= 3 && routed);
+  return few || some || rows >= 4096;
+}
+
+// several entries on the staged tiles, where tabs_pay says so: q8_gate_up (MATS 2) where tab_launch's shapes hold,
 // q8_group_tok (MATS 1) over whole workgroups of rows (false in *taken: not taken)
 template <uint32_t T, int L, int MATS>
-bool tabs_launch_l(const Args& a, int most, hipStream_t s, bool* taken) {
+bool tabs_launch_l(const Args& a, uint32_t max_cnt, hipStream_t s, bool* taken) {
   constexpr int NB = L == 16 ? 4 : 2, W = L == 16 || fused::grid_bytes<T>() >= 8192 ? 8 : 4, kT = kWave * W;
   using LD = fused::TabLds<T, L, NB, W, MATS>;
-  const uint32_t rb = (uint32_t) row_bytes<T>(a.cols), words = LD::R * rb / 16;
-  *taken = LD::total <= 64 * 1024 && a.rows % LD::R == 0 && (LD::R * rb) % 16 == 0 &&
-           words <= (uint32_t) fused::kG1Slots * kT && ((uintptr_t) a.q & 15) == 0;
-  if (!*taken) return false;
-  if constexpr (LD::total <= 64 * 1024) {
+  if constexpr (tabs_serve<T, L, MATS>() && LD::total <= 64 * 1024) {
+    const uint32_t rb = (uint32_t) row_bytes<T>(a.cols), words = LD::R * rb / 16;
+    *taken = a.rows % LD::R == 0 && (LD::R * rb) % 16 == 0 && words <= (uint32_t) fused::kG1Slots * kT &&
+             ((uintptr_t) a.q & 15) == 0 && tabs_pay<T, L, MATS>(a.n, max_cnt, a.rows, a.cols, a.n * (a.rows / LD::R));
+    if (!*taken) return false;
     fused::GuArgs ga{};
     ga.dim = a.cols, ga.ff = a.rows, ga.lim = a.lim;
+    const int most = max_cnt > 4 ? 8 : (int) max_cnt;  // (as the per-row kernels' token tiles)
     const fused::G1Tab tb = {(const uint8_t* const*) a.wg, (const uint8_t* const*) a.wu, a.cnt, a.xrow, a.xin, a.win,
                              a.q, a.d, a.scale, a.y, a.ys, most};
     const dim3 grid(a.rows / LD::R, a.n);
     if (words <= (uint32_t) kT) fused::tab_kernel<T, 1, L, NB, W, MATS><<<grid, kT, 0, s>>>(ga, tb);
     else if (words <= 2u * kT) fused::tab_kernel<T, 2, L, NB, W, MATS><<<grid, kT, 0, s>>>(ga, tb);
     else fused::tab_kernel<T, fused::kG1Slots, L, NB, W, MATS><<<grid, kT, 0, s>>>(ga, tb);
+    return hipGetLastError() == hipSuccess;
   }
-  return hipGetLastError() == hipSuccess;
+  return false;
 }
 template <uint32_t T, int MATS>
-bool tabs_launch(const Args& a, int most, hipStream_t s, bool* taken) {
+bool tabs_launch(const Args& a, uint32_t max_cnt, hipStream_t s, bool* taken) {
   *taken = false;
-  if (a.cols % 512 == 0 && a.cols <= fused::G1Max<16>::dim) return tabs_launch_l<T, 16, MATS>(a, most, s, taken);
-  if (a.cols % 1024 == 0 && a.cols >= 4096 && a.cols <= fused::G1Max<32>::dim) return tabs_launch_l<T, 32, MATS>(a, most, s, taken);
+  if (a.cols % 512 == 0 && a.cols <= fused::G1Max<16>::dim) return tabs_launch_l<T, 16, MATS>(a, max_cnt, s, taken);
+  if (a.cols % 1024 == 0 && a.cols >= 4096 && a.cols <= fused::G1Max<32>::dim) return tabs_launch_l<T, 32, MATS>(a, max_cnt, s, taken);
   return false;
 }
 
@@ -652,14 +690,9 @@ bool by_lanes(const Args& a, bool fused, hipStream_t s, uint32_t tiles = 1) {
 template <uint32_t T>
 bool by_tokens(const Args& a, uint32_t max_cnt, bool fused, hipStream_t s) {
   if (a.cols % Block<T>::values) return false;
-  // several tokens an entry, or one where the tile beats the per-row kernels (us a layer of 9 or 10 experts: 2048 -> 7168
-  // IQ3_XXS 93.9 -> 68.4, IQ1_S 61.5 -> 54.8, IQ1_M 66.0 -> 60.6, IQ2_XXS 74.2 -> 71.8; 512 -> 2048 IQ3_XXS 25.4 -> 24.9, the
-  // others slower). one matrix alone keeps the kernels above: they put more waves on it
-  constexpr bool kIq = T != kQ2_K && T != kQ4_0 && T != kQ4_K && T != kQ3_K;
-  if (a.n > 1 && (max_cnt > 1 || (!fused && kIq && (a.cols >= 1024 || T == kIQ3_XXS)))) {
+  if (a.n > 1) {  // (one matrix alone keeps the kernels below: they put more waves on it)
     bool taken = false;
-    const int most = max_cnt > 4 ? 8 : (int) max_cnt;  // (as the token tiles below)
-    const bool ok = fused ? tabs_launch<T, 2>(a, most, s, &taken) : tabs_launch<T, 1>(a, most, s, &taken);
+    const bool ok = fused ? tabs_launch<T, 2>(a, max_cnt, s, &taken) : tabs_launch<T, 1>(a, max_cnt, s, &taken);
     if (taken) return ok;
   }
   switch (max_cnt) {
