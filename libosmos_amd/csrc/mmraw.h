@@ -8,7 +8,8 @@
 // 4-byte header word 6.1). head() hands the words round between the lane groups (v_permlane16_swap, v_permlane32_swap)
 // and decodes the block's fields; step() gives the 8 f16 of one step.
 //
-// The values are decode.h's, rounded to f16 (nearest even): the same F32 products and sums, then one conversion. What an
+// The values are decode.h's, rounded to f16 (nearest even): exact F32 scales and products, then one conversion. (A group's
+// scale is d times an odd whole number, 2 s + 1, never s d + d / 2, which is no number where d is infinite and s is 0.) What an
 // instruction costs chose the forms (measured, cycles a wave64 instruction): v_fma_mixlo/hi_f16 9, permlane swaps 8.3,
 // fma, conversions, perm, bfi and packed f16 4.5, F32 mul / add, shifts and logic 2.6. No asm holds an instruction: the
 // compiler does not see into asm, and a VALU write needs idle states before a matrix instruction reads it.
@@ -290,12 +291,12 @@ template <> struct Raw<kIQ2_XXS> {
     spread4(r.n[1] ^ flip, x), spread4(r.n[3] ^ flip, y);
 #pragma unroll
     for (int i = 0; i < 4; i++) h.a[2 * i] = x[i], h.a[2 * i + 1] = y[i];
-    h.d = 0.25f * f16(r.d & 0x7FFFu);
+    h.d = 0.125f * f16(r.d & 0x7FFFu);
   }
   template <int NPW> __device__ static half8 step(const H<NPW>& h, const Tab<kIQ2_XXS>& tab, int j, int s, int q) {
     const int g = 4 * j + s;
     const uint4 v = tab.g[(h.t[g / 2] >> (8 * (g & 1))) & 255u];
-    const float S = __builtin_fmaf((float) (h.a[g] >> 28), h.d, 0.5f * h.d);
+    const float S = mul(h.d, (float) (h.a[g] >> 27 | 1u));  // (2 s + 1: the top four bits over a one)
     const uint32_t sw = sign_word(__builtin_amdgcn_ubfe(h.a[g], 7 * q, 7));
     // the group's three magnitudes, picked by the entry's selectors
     const uint32_t v01 = pk16(mul(S, 8.0f), mul(S, 25.0f)), v2 = pk16x2(mul(S, 43.0f));
@@ -324,12 +325,12 @@ template <> struct Raw<kIQ3_XXS> {
     spread4(r.a[0] ^ flip, x), spread4(r.a[1] ^ flip, y);
 #pragma unroll
     for (int i = 0; i < 4; i++) h.a[2 * i] = x[i], h.a[2 * i + 1] = y[i];
-    h.d = 0.5f * f16(r.d & 0x7FFFu);
+    h.d = 0.25f * f16(r.d & 0x7FFFu);
   }
   template <int NPW> __device__ static half8 step(const H<NPW>& h, const Tab<kIQ3_XXS>& tab, int j, int s, int q) {
     const int g = 4 * j + s;
     const uint2 v0 = tab.g[(h.t[g / 2] >> (16 * (g & 1))) & 255u], v1 = tab.g[(h.t[g / 2] >> (16 * (g & 1) + 8)) & 255u];
-    const float S = __builtin_fmaf((float) (h.a[g] >> 28), h.d, 0.5f * h.d);
+    const float S = mul(h.d, (float) (h.a[g] >> 27 | 1u));  // (2 s + 1: the top four bits over a one)
     const uint32_t sw = sign_word(__builtin_amdgcn_ubfe(h.a[g], 7 * q, 7));
     const uint32_t w[4] = {v0.x, v0.y, v1.x, v1.y};
     uint32_t o[4];
@@ -365,7 +366,7 @@ template <> struct Raw<kIQ1_S> {
     const int g = 4 * j + s, o = 16 * (g & 1);
     const uint32_t qh = h.h[g / 2];
     const uint32_t idx = ((h.t[g / 2] >> (8 * (g & 1))) & 255u) | __builtin_amdgcn_ubfe(qh, o + 3 * q, 3) << 8;
-    const float S = __builtin_fmaf((float) ((qh >> (o + 12)) & 7u), 2.0f * h.d, h.d);
+    const float S = mul(h.d, (float) (((qh >> (o + 11)) & 14u) | 1u));
     return iq1_pick(S, (qh >> (o + 15)) & 1u, tab.g[idx]);
   }
 };
@@ -388,15 +389,15 @@ template <> struct Raw<kIQ1_M> {
     uint32_t e = r.s, f = r.s;
     swap0(e, f);
     h.d = f16(((e >> 12) & 15u) | ((e >> 28) << 4) | ((f >> 12) & 15u) << 8 | (f >> 28) << 12);
-    const int sh = 3 * (q >> 1);
-    h.s[0] = e >> sh, h.s[1] = f >> sh;
+    const int sh = 3 * (q >> 1);  // (doubled: 2 s + 1 is what the steps read)
+    h.s[0] = (e << 1) >> sh, h.s[1] = (f << 1) >> sh;
   }
   template <int NPW> __device__ static half8 step(const H<NPW>& h, const Tab<kIQ1_M>& tab, int j, int s, int q) {
     const int g = 4 * j + s;
     const uint32_t nib = __builtin_amdgcn_ubfe(h.h[g / 2], 16 * (g & 1) + 4 * q, 4);
     const uint32_t idx = ((h.t[g / 2] >> (8 * (g & 1))) & 255u) | (nib & 7u) << 8;
-    const uint32_t sc = (h.s[g >> 2] >> (16 * ((g >> 1) & 1) + 6 * (g & 1))) & 7u;
-    const float S = __builtin_fmaf((float) sc, 2.0f * h.d, h.d);
+    const uint32_t sc = ((h.s[g >> 2] >> (16 * ((g >> 1) & 1) + 6 * (g & 1))) & 14u) | 1u;
+    const float S = mul(h.d, (float) sc);
     return iq1_pick(S, nib & 8u, tab.g[idx]);
   }
 };
