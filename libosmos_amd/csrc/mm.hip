@@ -343,17 +343,12 @@ __device__ inline f32x4 add4(f32x4 a, f32x4 b) {
 // before is decoded, x a step or more ahead (D steps), and nothing is shared until the end, where the waves add their
 // partitions in order, each onto the sums of the waves before it. few partitions a wave: many waves for a small launch;
 // a whole block's, and more rows and tokens: its decode and its x serve more products (x, not the weights, is most of
-// what a large launch reads)
+// what a large launch reads). t0: the pass's first token
 template <uint32_t T, int NPW, int RT, int CT, int RW, int D>
-__global__ __launch_bounds__(Raw<T>::W / NPW * RW * kWave) void split_kernel(Args a) {
+__device__ __forceinline__ void split_pass(const Args& a, const Job& J, uint32_t t0, f32x4* part, Tab<T>& tab) {
   using X = Raw<T>;
   constexpr int KW = X::W / NPW, SS = X::SL / 32, NS = NPW * SS;  // partition waves, steps a slab, the wave's steps a block
   constexpr int PB = X::NP / NPW, NB = X::W / X::NP;              // waves a block, block classes
-  __shared__ f32x4 part[KW > 1 ? RW * RT * CT * kWave : 1];
-  __shared__ Tab<T> tab;
-  const Job J = job_of(a);
-  const uint32_t t0 = blockIdx.z * kTile * CT;
-  if (t0 >= J.n) return;  // (uniform: the whole workgroup)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int kw = wave % KW, rg = wave / KW, q = lane / 16, pw = kw % PB * NPW;
   const uint32_t row0 = (blockIdx.x * RW + rg) * kTile * RT;
@@ -441,6 +436,30 @@ __global__ __launch_bounds__(Raw<T>::W / NPW * RW * kWave) void split_kernel(Arg
     if (k + 1 < KW) __syncthreads();
   }
 }
+template <uint32_t T, int NPW, int RT, int CT, int RW, int D>
+__global__ __launch_bounds__(Raw<T>::W / NPW * RW * kWave) void split_kernel(Args a) {
+  __shared__ f32x4 part[Raw<T>::W > NPW ? RW * RT * CT * kWave : 1];
+  __shared__ Tab<T> tab;
+  const Job J = job_of(a);
+  const uint32_t t0 = blockIdx.z * kTile * CT;
+  if (t0 >= J.n) return;  // (uniform: the whole workgroup)
+  split_pass<T, NPW, RT, CT, RW, D>(a, J, t0, part, tab);
+}
+// four token tiles a pass at most, by the matrix's own: the few-token experts of a routed launch hold and load no tile of the
+// busy ones (256 experts of 2048 x 7168, 512 tokens x 8, one launch, us: IQ2_XXS 815 -> 628, IQ1_S 814 -> 608, IQ3_XXS 987 ->
+// 807; 7168 x 2048 Q4_K 1317 -> 1180, Q3_K 1060 -> 907). held to 256 VGPRs: the three bodies together took more. (Q3_K without
+// the one for two tiles: 24 of 512 x 2048 at 150 tokens 31 us, 37 with it)
+template <uint32_t T, int NPW, int RT, int RW, int D>
+__global__ __launch_bounds__(Raw<T>::W / NPW * RW * kWave) __attribute__((amdgpu_waves_per_eu(2))) void own_kernel(Args a) {
+  __shared__ f32x4 part[Raw<T>::W > NPW ? RW * RT * 4 * kWave : 1];
+  __shared__ Tab<T> tab;
+  const Job J = job_of(a);
+  const uint32_t t0 = blockIdx.z * kTile * 4;
+  if (t0 >= J.n) return;  // (uniform)
+  if (J.n - t0 <= kTile) split_pass<T, NPW, RT, 1, RW, 4>(a, J, t0, part, tab);
+  else if (T != kQ3_K && J.n - t0 <= 2 * kTile) split_pass<T, NPW, RT, 2, RW, 2>(a, J, t0, part, tab);
+  else split_pass<T, NPW, RT, 4, RW, D>(a, J, t0, part, tab);
+}
 
 // 16 tokens at most and rows enough for the chip: a wave is one row tile over all of K, every partition's sums in its
 // registers (Q4_K: 16 of 4), so nothing meets at the end; the workgroup's RW waves share x through LDS, kXCols columns at
@@ -524,10 +543,17 @@ bool launch_split(const Args& a, uint32_t n_mat, uint32_t max_n, hipStream_t s) 
   split_kernel<T, NPW, RT, CT, RW, D><<<grid, Raw<T>::W / NPW * RW * kWave, 0, s>>>(a);
   return hipGetLastError() == hipSuccess;
 }
+template <uint32_t T, int NPW, int RT, int RW, int D>
+bool launch_own(const Args& a, uint32_t n_mat, uint32_t max_n, hipStream_t s) {
+  constexpr uint32_t rows = kTile * RT * RW;
+  const dim3 grid((a.rows + rows - 1) / rows, n_mat, (max_n + 4 * kTile - 1) / (4 * kTile));
+  own_kernel<T, NPW, RT, RW, D><<<grid, Raw<T>::W / NPW * RW * kWave, 0, s>>>(a);
+  return hipGetLastError() == hipSuccess;
+}
 template <uint32_t T>
 bool launch_direct(const Args& a, uint32_t n_mat, uint32_t max_n, hipStream_t s) {
   constexpr int S = split_of<T>(), NP = Raw<T>::NP;
-  const uint64_t tiles = (uint64_t) (a.rows / kTile) * n_mat;
+  const uint64_t tiles = (uint64_t) (a.rows / kTile) * n_mat, passes = tiles * ((max_n + 4 * kTile - 1) / (4 * kTile));
   if (max_n <= kTile) {
     if (tiles < kLarge1) return launch_split<T, S, 1, 1, 1, 4>(a, n_mat, max_n, s);
     constexpr int RW = sizeof(Tab<T>) > 16384 ? 8 : 4;  // (IQ1's 32 KB codebook: more waves a copy)
@@ -538,11 +564,11 @@ bool launch_direct(const Args& a, uint32_t n_mat, uint32_t max_n, hipStream_t s)
     if (tiles < kLarge2) return launch_split<T, S, 1, 2, 1, 2>(a, n_mat, max_n, s);
     return launch_split<T, NP, 2, 2, 2, 2>(a, n_mat, max_n, s);
   }
-  if (tiles * ((max_n + 4 * kTile - 1) / (4 * kTile)) < large4<T>()) return launch_split<T, S, 1, 4, 1, 2>(a, n_mat, max_n, s);
+  if (passes < large4<T>()) return launch_split<T, S, 1, 4, 1, 2>(a, n_mat, max_n, s);
   // (Q4_K's whole block and IQ3_XXS's four classes would spill at two row groups or eight partitions)
-  if constexpr (T == kQ4_K) return launch_split<T, 4, 2, 4, 1, 2>(a, n_mat, max_n, s);
-  else if constexpr (T == kIQ3_XXS) return launch_split<T, NP, 2, 4, 1, 2>(a, n_mat, max_n, s);
-  else return launch_split<T, NP, 2, 4, 2, 1>(a, n_mat, max_n, s);
+  constexpr int N4 = T == kQ4_K ? 4 : NP, RW4 = T == kQ4_K || T == kIQ3_XXS ? 1 : 2, D4 = 3 - RW4;
+  if (n_mat > 1) return launch_own<T, N4, 2, RW4, D4>(a, n_mat, max_n, s);
+  return launch_split<T, N4, 2, 4, RW4, D4>(a, n_mat, max_n, s);  // (one matrix: all its passes but the last are whole)
 }
 template <uint32_t T> constexpr bool direct() {
   return T == kQ4_0 || T == kQ3_K || T == kQ4_K || T == kIQ1_S || T == kIQ1_M || T == kIQ2_XXS || T == kIQ3_XXS;
