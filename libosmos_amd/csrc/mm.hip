@@ -352,7 +352,10 @@ __device__ __forceinline__ void split_pass(const Args& a, const Job& J, uint32_t
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
   const int kw = wave % KW, rg = wave / KW, q = lane / 16, pw = kw % PB * NPW;
   const uint32_t row0 = (blockIdx.x * RW + rg) * kTile * RT;
-  const int tiles = min((int) ((J.n - t0 + kTile - 1) / kTile), CT);
+  // (one tile is known to be live; said only for IQ1, 768 x 2048 of 32 experts, us, IQ1_M 18.7 -> 16.7, the other types' loops
+  // are scheduled the better with the test in them, IQ3_XXS 2048 x 7168 of 8 28.3, 29.6 without)
+  constexpr bool kKnown = CT == 1 && (T == kIQ1_S || T == kIQ1_M);
+  const int tiles = kKnown ? 1 : min((int) ((J.n - t0 + kTile - 1) / kTile), CT);
   const uint32_t rb = (uint32_t) row_bytes<T>(a.cols), nblk = a.cols / 256, blk0 = kw / PB;
   const uint8_t* wr[RT];
 #pragma unroll
@@ -529,12 +532,16 @@ __global__ __launch_bounds__(RW * kWave) void rows_kernel(Args a) {
 // and two row tiles. measured, us, split / whole: one 16-token tile, Q4_K 7168 x 2048: 896 row tiles 9.3 / 12.2, 1792
 // 15.9 / 14.0; IQ2_XXS 2048 x 7168: 1024 28.0 / 32.2, 2048 50.3 / 41.3. two: Q4_K 896 11.3 / 9.9, IQ2_XXS 512 18.0 / 29.4,
 // 1024 33.3 / 30.0. four: Q4_K 448 9.2 / 8.3, IQ3_XXS 384 24.1 / 23.2, Q3_K 448 10.6 / 13.8, 896 18.3 / 13.8, IQ2_XXS 512
-// 26.0 / 36.6
+// 26.0 / 36.6.
+// Q4_0, whose two partition waves read the same words, has a form between the two, whole blocks and one row tile (us, split or
+// whole / it, by row tiles x passes): one tile 384 9.3 / 9.2, 896 11.4 / 9.8, 1024 (2048 x 7168) 37.2 / 31.8, 1536 17.1 / 13.9,
+// 3584 30.3 / 30.3; two 448 9.2 / 11.3, 896 13.8 / 12.1, 1024 44.2 / 40.0, 1536 20.0 / 18.3, 3584 36.2 / 41.5; four 768 14.7 /
+// 15.4 (and 17.3 whole), 896 17.4 / 15.5, 1024 50.1 / 44.6, 1536 23.5 / 22.0, 1792 24.2 / 25.7
 template <uint32_t T> constexpr int split_of() {
   return T == kQ4_K ? 4 : T == kQ4_0 || T == kQ3_K || T == kIQ3_XXS ? 2 : 1;
 }
 constexpr uint64_t kLarge1 = 2048, kLarge2 = 896;
-template <uint32_t T> constexpr uint64_t large4() { return T == kQ4_K || T == kIQ3_XXS ? 384 : 768; }
+template <uint32_t T> constexpr uint64_t large4() { return T == kQ4_K || T == kIQ3_XXS ? 384 : T == kQ4_0 ? 832 : 768; }
 
 template <uint32_t T, int NPW, int RT, int CT, int RW, int D>
 bool launch_split(const Args& a, uint32_t n_mat, uint32_t max_n, hipStream_t s) {
@@ -554,6 +561,11 @@ template <uint32_t T>
 bool launch_direct(const Args& a, uint32_t n_mat, uint32_t max_n, hipStream_t s) {
   constexpr int S = split_of<T>(), NP = Raw<T>::NP;
   const uint64_t tiles = (uint64_t) (a.rows / kTile) * n_mat, passes = tiles * ((max_n + 4 * kTile - 1) / (4 * kTile));
+  if constexpr (T == kQ4_0) {
+    if (max_n <= kTile && tiles >= 320 && tiles < kLarge1) return launch_split<T, NP, 1, 1, 4, 4>(a, n_mat, max_n, s);
+    if (max_n > kTile && max_n <= 2 * kTile && tiles >= 768 && tiles < kLarge1) return launch_split<T, NP, 1, 2, 4, 2>(a, n_mat, max_n, s);
+    if (max_n > 2 * kTile && passes >= large4<T>() && passes < 1664) return launch_own<T, NP, 1, 2, 2>(a, n_mat, max_n, s);
+  }
   if (max_n <= kTile) {
     if (tiles < kLarge1) return launch_split<T, S, 1, 1, 1, 4>(a, n_mat, max_n, s);
     constexpr int RW = sizeof(Tab<T>) > 16384 ? 8 : 4;  // (IQ1's 32 KB codebook: more waves a copy)

@@ -1,5 +1,5 @@
-"""The direct f16 kernels where a launch's matrices hold different counts: each matrix runs the body of its own token
-tiles. Each form gives a token the bits it has alone (which
+"""The direct f16 kernels where a launch's matrices hold different counts: each matrix runs the body of its own token tiles, and
+Q4_0 has a form of its own between the small and the large launches. Each form gives a token the bits it has alone (which
 test_mm_direct_gpu.py holds to the oracle's order): no tolerance."""
 import numpy as np
 import pytest
@@ -26,7 +26,8 @@ def test_counts(g, name, cols):
     one = np.concatenate([run(g, name, w, rows, cols, mm_x16(g, x[i:i + 1])[0], 1) for i in range(n)])
     x16, _ = mm_x16(g, x)
     wd = g.dev(w)
-    for tiles, most in [(900, 40), (900, 70)]:  # (row tiles, most)
+    # (row tiles, most): Q4_0's middle form at one, two and four tiles, then large launches of two passes
+    for tiles, most in [(330, 16), (801, 32), (450, 70), (900, 40), (900, 70)]:
         cnt, y = group(g, t, wd, rows, cols, x16, n, tiles, most, tiles + most)
         assert (g.bits(y) == g.bits(np.concatenate([one[:c] for c in cnt]))).all(), (tiles, most)
 
