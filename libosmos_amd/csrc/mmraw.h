@@ -64,7 +64,8 @@ __device__ inline half2v code_pair(uint32_t w, int hi, half2v c) {
   return __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, w, hi ? 0x07030602u : 0x05010400u)) + c;
 }
 // 4 f16 pairs times an F32 scale, the products exact in F32, rounded once: the mixed fma to F32 (plus -0, so that a -0
-// product stays -0) and the packed conversion
+// product stays -0) and the packed conversion, or (Mixed) the mixed fma to f16
+template <bool Mixed = false>
 __device__ inline half8 scaled8(float s, const uint32_t* w) {
   float z = -0.0f;
   asm("" : "+s"(z));
@@ -73,7 +74,7 @@ __device__ inline half8 scaled8(float s, const uint32_t* w) {
   for (int i = 0; i < 4; i++) {
     const half2v g = __builtin_bit_cast(half2v, w[i]);
     float a = __builtin_fmaf(s, (float) g[0], z), b = __builtin_fmaf(s, (float) g[1], z);
-    asm("" : "+v"(a), "+v"(b));  // (held in F32: the f16 mixed fma is the slower)
+    if constexpr (!Mixed) asm("" : "+v"(a), "+v"(b));  // (held in F32: the f16 mixed fma is the slower)
     o[2 * i] = (_Float16) a, o[2 * i + 1] = (_Float16) b;
   }
   return o;
