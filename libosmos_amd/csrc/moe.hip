@@ -14,6 +14,8 @@
 
 #include "common.h"
 
+#include <type_traits>
+
 #include "x16.h"
 
 extern "C" {
@@ -285,8 +287,8 @@ __global__ __launch_bounds__(256) void moe_sum_kernel(const float* __restrict__ 
 }
 
 // the same with a thread 4 values and blockIdx.y the token (dim a multiple of 4, 16-aligned rows): the picks' rows loaded
-// 8 at a time before their products are added in order. HBM-bound: 512 tokens x 8 picks of 7168 (147 MB) 64 -> 24 us
-constexpr int kSumPicks = 8;
+// N at a time before their products are added in order. HBM-bound: 512 tokens x 8 picks of 7168 (147 MB) 64 -> 24 us
+template <int N>
 __global__ __launch_bounds__(256) void moe_sum4_kernel(const float* __restrict__ y, const int32_t* __restrict__ where,
                                                        const float* __restrict__ w, uint32_t k, uint32_t dim,
                                                        const float* __restrict__ shared,
@@ -294,17 +296,17 @@ __global__ __launch_bounds__(256) void moe_sum4_kernel(const float* __restrict__
   const uint32_t t = blockIdx.y, d = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (d >= dim) return;
   float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (uint32_t j0 = 0; j0 < k; j0 += kSumPicks) {
-    const uint32_t n = min(k - j0, (uint32_t) kSumPicks);
-    float4 v[kSumPicks];
-    float wj[kSumPicks];
+  for (uint32_t j0 = 0; j0 < k; j0 += N) {
+    const uint32_t n = min(k - j0, (uint32_t) N);
+    float4 v[N];
+    float wj[N];
 #pragma unroll
-    for (uint32_t j = 0; j < kSumPicks; j++) {  // (past the picks: the last again, not added)
+    for (uint32_t j = 0; j < N; j++) {  // (past the picks: the last again, not added)
       const uint32_t at = t * k + j0 + min(j, n - 1);
       v[j] = *(const float4*) (y + (uint64_t) where[at] * dim + d), wj[j] = w[at];
     }
 #pragma unroll
-    for (uint32_t j = 0; j < kSumPicks; j++)
+    for (uint32_t j = 0; j < N; j++)
       if (j < n) {  // (uniform)
         s[0] = __fadd_rn(s[0], __fmul_rn(v[j].x, wj[j])), s[1] = __fadd_rn(s[1], __fmul_rn(v[j].y, wj[j]));
         s[2] = __fadd_rn(s[2], __fmul_rn(v[j].z, wj[j])), s[3] = __fadd_rn(s[3], __fmul_rn(v[j].w, wj[j]));
@@ -408,8 +410,9 @@ __global__ __launch_bounds__(256) void copy_rows_kernel(float* __restrict__ dst,
 }
 
 // y[t][d] = sum over j in order of src[idx[t m + j]][d] (from 0), then add's (kernels/ops.hip:515-525); a thread a value,
-// its rows' values loaded 8 at a time before they are added (one at a time, each load waited for the index and the row
+// its rows' values loaded N at a time before they are added (one at a time, each load waited for the index and the row
 // before it: 4 tokens x 10 rows of 2048 6.2 -> 4.5 us)
+template <int N>
 __global__ __launch_bounds__(256) void gather_sum_kernel(float* __restrict__ y, const float* __restrict__ src,
                                                          const int32_t* __restrict__ idx, uint32_t m, uint32_t n,
                                                          uint32_t dim, const float* __restrict__ add) {
@@ -417,14 +420,14 @@ __global__ __launch_bounds__(256) void gather_sum_kernel(float* __restrict__ y, 
   if (i >= (uint64_t) n * dim) return;
   const uint32_t t = (uint32_t) (i / dim), d = (uint32_t) (i % dim);
   float s = 0.0f;
-  for (uint32_t j0 = 0; j0 < m; j0 += kSumPicks) {
-    const uint32_t left = min(m - j0, (uint32_t) kSumPicks);
-    float v[kSumPicks];
+  for (uint32_t j0 = 0; j0 < m; j0 += N) {
+    const uint32_t left = min(m - j0, (uint32_t) N);
+    float v[N];
 #pragma unroll
-    for (uint32_t j = 0; j < kSumPicks; j++)  // (past the rows: the last again, not added)
+    for (uint32_t j = 0; j < N; j++)  // (past the rows: the last again, not added)
       v[j] = src[(uint64_t) idx[t * m + j0 + min(j, left - 1)] * dim + d];
 #pragma unroll
-    for (uint32_t j = 0; j < kSumPicks; j++)
+    for (uint32_t j = 0; j < N; j++)
       if (j < left) s = __fadd_rn(s, v[j]);
   }
   y[i] = add ? __fadd_rn(s, add[i]) : s;
@@ -515,6 +518,16 @@ __global__ __launch_bounds__(kLaneThreads) void lane_tables_kernel(const int32_t
     for (uint32_t j = t0; j < t0 + k; j++) place += row_of[j] < r;
     order[t0 + place] = r;
   }
+}
+
+// f(the rows in flight of a sum of k). past a short sum's last row the kernels load it again: at 8 always, 512 tokens of one row
+// of 4096 took 8.7 us (5.7 one at a time), and the shortest calls 0.1 to 0.3 us more
+template <typename F>
+inline void by_rows(uint32_t k, F f) {
+  if (k == 1) f(std::integral_constant<int, 1>{});
+  else if (k == 2) f(std::integral_constant<int, 2>{});
+  else if (k <= 4) f(std::integral_constant<int, 4>{});
+  else f(std::integral_constant<int, 8>{});
 }
 
 inline unsigned grid256(uint64_t n) { return (unsigned) ((n + 255) / 256); }
@@ -626,8 +639,10 @@ extern "C" OSM_API bool q4x_moe_sum(const float* y, const int32_t* where, const 
                                     void* stream) {
   if (!y || !where || !w || !shared || !shared_logit || !out || !n_tok || !k || !dim) return false;
   if (dim % 4 == 0 && n_tok <= moe::kGridY && moe::aligned16(y, shared, out)) {
-    moe::moe_sum4_kernel<<<dim3((dim + 1023) / 1024, n_tok), 256, 0, (hipStream_t) stream>>>(y, where, w, k, dim, shared,
-                                                                                            shared_logit, out);
+    moe::by_rows(k, [&](auto n) {
+      moe::moe_sum4_kernel<decltype(n)::value><<<dim3((dim + 1023) / 1024, n_tok), 256, 0, (hipStream_t) stream>>>(
+          y, where, w, k, dim, shared, shared_logit, out);
+    });
     return hipGetLastError() == hipSuccess;
   }
   moe::moe_sum_kernel<<<moe::grid256((uint64_t) n_tok * dim), 256, 0, (hipStream_t) stream>>>(y, where, w, n_tok, k, dim,
@@ -700,7 +715,10 @@ extern "C" OSM_API bool ops_copy_rows(float* dst, const float* src, const int32_
 extern "C" OSM_API bool ops_gather_sum_add(float* y, const float* src, const int32_t* idx, uint32_t m, uint32_t n,
                                            uint32_t dim, const float* add, void* stream) {
   if (!y || !src || !idx || !m || !n || !dim || !add) return false;
-  moe::gather_sum_kernel<<<moe::grid256((uint64_t) n * dim), 256, 0, (hipStream_t) stream>>>(y, src, idx, m, n, dim, add);
+  moe::by_rows(m, [&](auto r) {
+    moe::gather_sum_kernel<decltype(r)::value><<<moe::grid256((uint64_t) n * dim), 256, 0, (hipStream_t) stream>>>(
+        y, src, idx, m, n, dim, add);
+  });
   return hipGetLastError() == hipSuccess;
 }
 

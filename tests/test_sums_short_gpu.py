@@ -1,0 +1,34 @@
+"""Sums of 1 to 9 rows (1, 2, 4 or 8 in flight), bit for bit numpy's float32 steps in the contract's order."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def g():
+    import torch  # noqa: F401
+    from tests import gpu_util
+    return gpu_util
+
+
+@pytest.mark.parametrize("k", range(1, 10))
+@pytest.mark.parametrize("dim", [5, 260])
+def test_sums(g, k, dim):
+    import torch
+    rng = np.random.default_rng(k)
+    n_tok, rows = 3, 3 * k
+    y, sh = (rng.normal(0, 1, s).astype(np.float32) for s in ((rows, dim), (n_tok, dim)))
+    where, w = rng.permutation(rows).astype(np.int32), rng.uniform(0, 1, rows).astype(np.float32)
+    yd, wh, shd = g.dev(y), g.dev(where), g.dev(sh)
+    out = torch.full((n_tok, dim), float("nan"), device="cuda")
+    print("sums", dim, k, flush=True)
+    g.call("q4x_moe_sum", g.a(yd), g.a(wh), g.a(g.dev(w)), n_tok, k, dim, g.a(shd), g.a(g.dev(np.zeros(n_tok, np.float32))),
+           g.a(out), None)
+    want, plain = np.zeros((n_tok, dim), np.float32), np.zeros((n_tok, dim), np.float32)
+    for j in range(k):
+        r = where.reshape(n_tok, k)[:, j]
+        want, plain = want + y[r] * w.reshape(n_tok, k)[:, j:j + 1], plain + y[r]
+    assert (g.bits(g.host(out)) == g.bits(want + sh * np.float32(0.5))).all()  # (the gate at a zero logit: exactly 1/2)
+    g.call("ops_gather_sum_add", g.a(out), g.a(yd), g.a(wh), k, n_tok, dim, g.a(shd), None)
+    assert (g.bits(g.host(out)) == g.bits(plain + sh)).all()
