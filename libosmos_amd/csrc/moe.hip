@@ -288,6 +288,7 @@ __global__ __launch_bounds__(256) void moe_sum_kernel(const float* __restrict__ 
 
 // the same with a thread 4 values and blockIdx.y the token (dim a multiple of 4, 16-aligned rows): the picks' rows loaded
 // N at a time before their products are added in order. HBM-bound: 512 tokens x 8 picks of 7168 (147 MB) 64 -> 24 us
+constexpr uint32_t kGridY = 65535;  // blockIdx.y's most
 template <int N>
 __global__ __launch_bounds__(256) void moe_sum4_kernel(const float* __restrict__ y, const int32_t* __restrict__ where,
                                                        const float* __restrict__ w, uint32_t k, uint32_t dim,
@@ -360,15 +361,19 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(float* __restrict__ ds
   if (i < (uint64_t) n * len) dst[i] = src[(uint64_t) idx[i / len] * len + i % len];
 }
 
-// the same with a thread 4 values and blockIdx.y a row (len a multiple of 4, 16-aligned rows; rows past the grid's most by
-// strides): 4096 rows of 7168 (117 MB written) 60 -> 35 us
-constexpr uint32_t kGridY = 65535;
-__global__ __launch_bounds__(256) void gather_rows4_kernel(float* __restrict__ dst, const float* __restrict__ src,
-                                                           const int32_t* __restrict__ idx, uint32_t n, uint32_t len) {
-  const uint32_t c = (blockIdx.x * 256 + threadIdx.x) * 4;
-  if (c >= len) return;
-  for (uint32_t r = blockIdx.y; r < n; r += gridDim.y)
-    *(float4*) (dst + (uint64_t) r * len + c) = *(const float4*) (src + (uint64_t) idx[r] * len + c);
+// the same with a thread 4 values (len a multiple of 4, 16-aligned rows): 4096 rows of 7168 (117 MB written) 60 -> 35 us. words:
+// the rows' words, a thread each; Many: past a launch's most threads, each further ones by strides (a multiply and a divide
+// of 64 bits)
+constexpr uint64_t kGatherThreads = 1u << 30;
+template <bool Many>
+__global__ __launch_bounds__(256) void gather_rows4_kernel(float4* __restrict__ dst, const float4* __restrict__ src,
+                                                           const int32_t* __restrict__ idx, uint64_t words, uint32_t per) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if constexpr (Many) {
+    for (uint64_t w = i; w < words; w += kGatherThreads) dst[w] = src[(uint64_t) idx[w / per] * per + w % per];
+  } else {
+    if (i < (uint32_t) words) dst[i] = src[(uint64_t) idx[i / per] * per + i % per];
+  }
 }
 
 // the stream held until *flag (host memory the GPU maps) holds value, with or without its top bit (the host's mark of
@@ -662,8 +667,10 @@ extern "C" OSM_API bool ops_gather_rows(float* dst, const float* src, const int3
                                         void* stream) {
   if (!dst || !src || !idx || !n || !len) return false;
   if (len % 4 == 0 && moe::aligned16(dst, src, nullptr)) {
-    moe::gather_rows4_kernel<<<dim3((len + 1023) / 1024, n < moe::kGridY ? n : moe::kGridY), 256, 0, (hipStream_t) stream>>>(
-        dst, src, idx, n, len);
+    const uint64_t words = (uint64_t) n * (len / 4);
+    auto* kernel = words > moe::kGatherThreads ? moe::gather_rows4_kernel<true> : moe::gather_rows4_kernel<false>;
+    kernel<<<moe::grid256(words < moe::kGatherThreads ? words : moe::kGatherThreads), 256, 0, (hipStream_t) stream>>>(
+        (float4*) dst, (const float4*) src, idx, words, len / 4);
     return hipGetLastError() == hipSuccess;
   }
   moe::gather_rows_kernel<<<moe::grid256((uint64_t) n * len), 256, 0, (hipStream_t) stream>>>(dst, src, idx, n, len);

@@ -1,4 +1,5 @@
-"""Sums of 1 to 9 rows (1, 2, 4 or 8 in flight), bit for bit numpy's float32 steps in the contract's order."""
+"""Sums of 1 to 9 rows (1, 2, 4 or 8 in flight), copies of short rows and one of more words than a launch's threads: bit for bit
+numpy's float32 steps in the contract's order."""
 import numpy as np
 import pytest
 
@@ -32,3 +33,31 @@ def test_sums(g, k, dim):
     assert (g.bits(g.host(out)) == g.bits(want + sh * np.float32(0.5))).all()  # (the gate at a zero logit: exactly 1/2)
     g.call("ops_gather_sum_add", g.a(out), g.a(yd), g.a(wh), k, n_tok, dim, g.a(shd), None)
     assert (g.bits(g.host(out)) == g.bits(plain + sh)).all()
+
+
+@pytest.mark.parametrize("n,dim", [(1, 4), (300, 4), (257, 12), (33, 256), (5, 1020), (5, 1028)])
+def test_rows(g, n, dim):
+    import torch
+    rng = np.random.default_rng(n)
+    y, idx = rng.normal(0, 1, (40, dim)).astype(np.float32), rng.integers(0, 40, n).astype(np.int32)
+    dst = torch.full((n, dim), float("nan"), device="cuda")
+    print("rows", n, dim, flush=True)
+    g.call("ops_gather_rows", g.a(dst), g.a(g.dev(y)), g.a(g.dev(idx)), n, dim, None)
+    assert (g.bits(g.host(dst)) == g.bits(y[idx])).all()
+
+
+def test_rows_by_strides(g):
+    import torch
+    n, dim = (1 << 22) + 3, 1024  # (2^30 + 768 words)
+    if torch.cuda.mem_get_info()[0] < 20e9:
+        pytest.skip("needs 17 GB of device memory")
+    src = torch.randn(7, dim, device="cuda")
+    idx = (torch.arange(n, device="cuda") % 7).to(torch.int32)
+    dst = torch.empty(n, dim, device="cuda")
+    at = torch.tensor([0, 1, (1 << 21) - 1, 1 << 21, (1 << 22) - 1, 1 << 22, n - 1], device="cuda")
+    dst[at] = 0.0
+    print("rows by strides", flush=True)
+    g.call("ops_gather_rows", g.a(dst), g.a(src), g.a(idx), n, dim, None)
+    assert torch.equal(dst[at], src[at % 7])
+    del dst
+    torch.cuda.empty_cache()
