@@ -538,16 +538,18 @@ inline void by_rows(uint32_t k, F f) {
 inline unsigned grid256(uint64_t n) { return (unsigned) ((n + 255) / 256); }
 inline bool aligned16(const void* a, const void* b, const void* c) { return (((uintptr_t) a | (uintptr_t) b | (uintptr_t) c) & 15) == 0; }
 
-// ---- q4x_swiglu_rows (kernels/q4x_moe.hip:235-253): a thread 8 columns of a slot in x16's own order (mm.hip's x16_kernel),
-// silu(g) u (swiglu_kernel's expression) rounded to f16 as mm_x16_rows rounds. Vec: g and u 16-byte aligned (7936 slots
-// of 2048, 99 MB: 69 -> 22 us) ----
-template <bool Vec>
+// ---- q4x_swiglu_rows (kernels/q4x_moe.hip:235-253): a thread 8 columns of a slot, silu(g) u (swiglu_kernel's expression)
+// rounded to f16 as mm_x16_rows rounds. Tiled: in x16's own order (mm.hip's x16_kernel), so that a wave stores side by side;
+// not for the few slots of up to two tiles, where a wave would hold few live threads (1 slot of 512: 3.1 us, 3.9 tiled). Vec: g
+// and u 16-byte aligned (7936 slots of 2048, 99 MB: 69 -> 22 us) ----
+template <bool Vec, bool Tiled>
 __global__ __launch_bounds__(256) void swiglu_rows_kernel(const float* __restrict__ g, const float* __restrict__ u,
                                                           uint32_t ff, const int32_t* __restrict__ idx, uint32_t slots,
                                                           _Float16* __restrict__ x16, int32_t* __restrict__ overflow) {
   const uint64_t i = (uint64_t) blockIdx.x * 256 + threadIdx.x;
-  const uint32_t frag = (uint32_t) (i / 32), per = ff / kX16Tile;
-  const uint32_t sl = frag / per * kX16Tile + (uint32_t) (i % 32) / 2, c = frag % per * kX16Tile + (uint32_t) (i % 2) * 8;
+  const uint32_t part = (uint32_t) (i / 32), per = ff / kX16Tile, groups = ff / 8;
+  const uint32_t sl = Tiled ? part / per * kX16Tile + (uint32_t) (i % 32) / 2 : (uint32_t) i / groups;
+  const uint32_t c = Tiled ? part % per * kX16Tile + (uint32_t) (i % 2) * 8 : (uint32_t) i % groups * 8;
   if (sl >= slots) return;
   const int32_t r = idx[sl];
   typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -566,7 +568,7 @@ __global__ __launch_bounds__(256) void swiglu_rows_kernel(const float* __restric
   }
 #pragma unroll
   for (int j = 0; j < 8; j++) h[j] = x16_round(r >= 0 ? __fmul_rn(silu(gv[j]), uv[j]) : 0.0f, over);
-  *(half8*) (x16 + i * 8) = h;
+  *(half8*) (x16 + (Tiled ? i * 8 : x16_at(sl, c, ff))) = h;
   if (over) *overflow = 1;
 }
 
@@ -630,12 +632,11 @@ extern "C" OSM_API bool q4x_spin(uint32_t us, void* stream) {
 extern "C" OSM_API bool q4x_swiglu_rows(const float* g, const float* u, uint32_t ff, const int32_t* idx,
                                         uint32_t slots, void* x16, int32_t* overflow, void* stream) {
   if (!g || !u || !idx || !x16 || (uintptr_t) x16 % 16 || !overflow || !slots || !ff || ff % kX16Tile) return false;
-  const uint64_t threads = (uint64_t) (slots + moe::kTile - 1) / moe::kTile * moe::kTile * (ff / 8);
-  const uint32_t grid = (uint32_t) ((threads + 255) / 256);
-  if (moe::aligned16(g, u, nullptr))
-    moe::swiglu_rows_kernel<true><<<grid, 256, 0, (hipStream_t) stream>>>(g, u, ff, idx, slots, (_Float16*) x16, overflow);
-  else
-    moe::swiglu_rows_kernel<false><<<grid, 256, 0, (hipStream_t) stream>>>(g, u, ff, idx, slots, (_Float16*) x16, overflow);
+  const bool tiled = slots > 2 * moe::kTile, vec = moe::aligned16(g, u, nullptr);
+  const uint64_t threads = (uint64_t) (tiled ? (slots + moe::kTile - 1) / moe::kTile * moe::kTile : slots) * (ff / 8);
+  auto* kernel = tiled ? (vec ? moe::swiglu_rows_kernel<true, true> : moe::swiglu_rows_kernel<false, true>)
+                       : (vec ? moe::swiglu_rows_kernel<true, false> : moe::swiglu_rows_kernel<false, false>);
+  kernel<<<(uint32_t) ((threads + 255) / 256), 256, 0, (hipStream_t) stream>>>(g, u, ff, idx, slots, (_Float16*) x16, overflow);
   return hipGetLastError() == hipSuccess;
 }
 

@@ -1,5 +1,6 @@
-"""Sums of 1 to 9 rows (1, 2, 4 or 8 in flight), copies of short rows and one of more words than a launch's threads: bit for bit
-numpy's float32 steps in the contract's order."""
+"""The MoE plumbing's short forms: sums of 1 to 9 rows (1, 2, 4 or 8 in flight), copies of short rows and one of more words
+than a launch's threads, SwiGLU rows of up to two tiles and just past them. Bit for bit numpy's float32 steps in the contract's order; the
+SwiGLU's bytes are those of the same rows among many, which test_plumbing_gpu.py holds to a bound."""
 import numpy as np
 import pytest
 
@@ -61,3 +62,24 @@ def test_rows_by_strides(g):
     assert torch.equal(dst[at], src[at % 7])
     del dst
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("n", [1, 3, 16, 17, 32, 33])
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("ff", [16, 528])
+def test_swiglu_rows(g, n, off, ff):
+    import torch
+    rng = np.random.default_rng(n + ff)
+    gg, uu = (rng.normal(0, 2, n * ff).astype(np.float32) for _ in range(2))
+    gd, ud = (torch.from_numpy(np.concatenate([np.zeros(off, np.float32), a])).cuda()[off:] for a in (gg, uu))
+    idx = rng.integers(-1, n, n).astype(np.int32)
+    print("swiglu", n, off, ff, flush=True)
+
+    def rows(ids):
+        slots = (len(ids) + 15) // 16 * 16
+        y = torch.full((slots * ff,), 7.0, dtype=torch.float16, device="cuda")
+        ov = torch.zeros(1, dtype=torch.int32, device="cuda")
+        g.call("q4x_swiglu_rows", g.a(gd), g.a(ud), ff, g.a(g.dev(ids)), len(ids), g.a(y), g.a(ov), None)
+        return g.host(y).view(np.uint16).reshape(-1, ff // 16, 16, 16).transpose(0, 2, 1, 3).reshape(-1, ff)
+    one, many = rows(idx), rows(np.concatenate([idx, np.zeros(64, np.int32)]))
+    assert (one[:n] == many[:n]).all() and (one[n:] == np.float16(7.0).view(np.uint16)).all()
