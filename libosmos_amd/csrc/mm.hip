@@ -14,6 +14,7 @@
 #include <type_traits>
 
 #include "mmraw.h"
+#include "mmstage.h"
 #include "x16.h"
 
 extern "C" {
@@ -186,7 +187,7 @@ __global__ __launch_bounds__(W * kWave) void kernel(Args a) {
   uint32_t woff[kPer];
 #pragma unroll
   for (uint32_t u = 0; u < kPer; u++) {
-    const uint32_t i = min(u * kThreads + threadIdx.x, kWords - 1);
+    const uint32_t i = stage_word(u, kThreads, threadIdx.x, kWords);
     if constexpr (kTiled) woff[u] = min(row0 / kTile + i / kWt, a.rows / kTile - 1) * kTile * rb + (i % kWt) * WB;
     else woff[u] = min(row0 + i / kWr, a.rows - 1) * rb + (i % kWr) * WB;
   }
@@ -201,10 +202,8 @@ __global__ __launch_bounds__(W * kWave) void kernel(Args a) {
       const uint32_t lim = (a.cols - r * kRv) / Block<T>::values * Block<T>::bytes;  // the round's bytes a row
       const uint8_t* base = w + (uint64_t) r * kRb;
 #pragma unroll
-      for (uint32_t u = 0; u < kPer; u++) {
-        const uint32_t o = min(u * kThreads + threadIdx.x, kWords - 1) % kWr * WB;  // (woff's word)
-        wr[u] = gload<word>(base + woff[u] - (o < lim ? 0 : o - (lim - WB)));  // (past a short round: its last word)
-      }
+      for (uint32_t u = 0; u < kPer; u++)
+        wr[u] = gload<word>(base + woff[u] - stage_back(stage_word(u, kThreads, threadIdx.x, kWords), kWr, WB, lim));
     }
   };
   auto store = [&](int buf) __attribute__((always_inline)) {

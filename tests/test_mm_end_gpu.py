@@ -1,7 +1,6 @@
-"""the staged f16 kernel on a matrix that ends where its memory does, at widths that leave its last round short: a
-workgroup's threads past the staged words read the last word again, inside the matrix. (They took a short round's step
-back from their own place instead of that word's, and read up to a round past the last row.) The buffer is a whole number of
-2 MiB pages with the matrix at its end; the bits are those of the matrix in the middle of one."""
+"""the staged f16 kernel on a matrix that ends where its memory does, at widths that leave its last round short: the bits are
+those of the matrix in the middle of the buffer, a whole number of 2 MiB pages. What the threads past the staged words read is
+never stored and shows in no bits: test_mm_stage.py checks that it lies inside the matrix."""
 import numpy as np
 import pytest
 
