@@ -16,9 +16,8 @@
 // in its own registers, and its results are tokens 4 (l / 16) + i. so a lane needs 4 tokens' dx and sx a group, and they
 // reach it as DPP operands (row_newbcast: a value of a lane of its row of 16) with no LDS read: the lane holds a
 // float a tile and 64 slots of dx, and one of sx. what bounds it is the epilogue - mul, fma, fma and a conversion a
-// result and group, 16 results an MFMA's 8 cycles - so the last tile of an expert's tokens spends it only on the
-// results i that hold a token (the tokens of a tile are laid out over the lanes as 4 i + l / 16, so that 5 tokens are 2
-// results of 4).
+// result and group, 16 results an MFMA's 8 cycles - so a pass of at most 8 tokens spends it only on the results i that hold
+// a token (the tokens of a tile are laid out over the lanes as 4 i + l / 16, so that 5 tokens are 2 results of 4).
 #include "mmraw.h"
 
 extern "C" {
@@ -169,8 +168,10 @@ struct QArgs {
 // them: one barrier a block. the weights' codes and header words come straight from global memory (mmraw.h's Q4_K).
 // with the rows as A (their scales and the tokens' dx, sx through LDS, two barriers a block) and so, us, x8_rows
 // included: 256 experts of 7168 x 2048, 512 tokens x 8: 875, 795; 128 of 2048 x 768: 148, 124; one expert of 17 tokens
-// 22.5, 15.5, of 512 53.6, 52.2; 64 of 1040 x 1024 at 40 tokens 21.6, 19.0; 16 of 2048 x 768 at 100 tokens 18.9, 19.8
-// (149 VGPRs hold 3 waves a SIMD where 4 were: its workgroups just miss one round of the chip; at 30 tokens 14.0, 12.4).
+// 22.5, 15.5, of 512 53.6, 52.2; 64 of 1040 x 1024 at 40 tokens 21.6, 19.0. slower, by up to 9 % (kernel alone, weights from
+// HBM), are short rows in launches of about one round of the chip, where 149 VGPRs hold 3 waves a SIMD and 4 were held: 16 of
+// 2048 x 768 at 40 / 64 / 100 / 200 tokens 13.5 / 16.3 / 23.4 / 36.3, 14.4 / 16.7 / 23.0 / 38.6. (held to 128 VGPRs, 5 spilled:
+// 13.6 / 17.3 / 23.2 / 38.0, but 240 of 383 launches slower, by 8 % in the mean.)
 // the kernel alone about 745, of which about 470 are left without the MFMAs and 555 without the loads: the epilogue's
 // VALU work, then its waits on the MFMAs
 template <int CT>
@@ -187,7 +188,7 @@ __global__ __launch_bounds__(kThreads) void q4k_kernel(QArgs a) {
   float* y = a.ya + a.yoff[m];
   const uint32_t soff = a.soff[m];
   auto pass = [&](auto tiles, auto results, uint32_t c0) __attribute__((always_inline)) {
-    constexpr int C = decltype(tiles)::value, NI = decltype(results)::value;  // tiles; the last one's results with tokens
+    constexpr int C = decltype(tiles)::value, NI = decltype(results)::value;  // tiles; a tile's results with tokens
     constexpr uint32_t XW = C * kXWords, DW = C * kDWords, XP = (XW + kThreads - 1) / kThreads, DP = (2 * DW + kThreads - 1) / kThreads;
     const uint32_t s0 = soff + c0;  // the pass's first slot: a multiple of 16
     u32x4 xr[XP];
@@ -256,8 +257,7 @@ __global__ __launch_bounds__(kThreads) void q4k_kernel(QArgs a) {
           for (int ct = 0; ct < C; ct++) {
             const long xv = *(const long*) (xb + ct * (int) kXWords * 16 + g * (MMQ_SLOTS * MMQ_GROUP));
             const v4i I = __builtin_amdgcn_mfma_i32_16x16x32_i8(xv, wv, v4i{0, 0, 0, 0}, 0, 0, 0);
-            if (ct == C - 1) qstep<NI, g % 4>(acc[p][ct], I, dv[ct][g / 4], sv[ct][g / 4], S, M);
-            else qstep<4, g % 4>(acc[p][ct], I, dv[ct][g / 4], sv[ct][g / 4], S, M);
+            qstep<NI, g % 4>(acc[p][ct], I, dv[ct][g / 4], sv[ct][g / 4], S, M);
           }
         };
         group(std::integral_constant<int, 0>{}), group(std::integral_constant<int, 1>{});

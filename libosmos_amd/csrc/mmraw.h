@@ -147,7 +147,7 @@ __device__ inline void fill_step_tab(Tab<T>& t) {  // every thread of the workgr
 // step's j: the partition - kPart: of the wave's, else of the block - and s its step of 32 values ----
 template <uint32_t T> struct Raw;
 // Q4_K: lane group q loads header word q and, of a whole block, group pair q's 32 bytes (four 8-byte units: unit u is what
-// lane group u decodes); of half a block 16 bytes; of a pair its own unit
+// lane group u decodes); of half a block 16 bytes
 template <> struct Raw<kQ4_K> {
   static constexpr int SL = 32, W = 16, NP = 8;
   static constexpr bool kPart = true;
@@ -157,12 +157,10 @@ template <> struct Raw<kQ4_K> {
     if constexpr (NPW == 8) {
       const W4 u = gload<W4>(b + 16 + 32 * q), v = gload<W4>(b + 32 + 32 * q);
       r.n[0] = u.x, r.n[1] = u.y, r.n[2] = u.z, r.n[3] = u.w, r.n[4] = v.x, r.n[5] = v.y, r.n[6] = v.z, r.n[7] = v.w;
-    } else if constexpr (NPW == 4) {
+    } else {
+      static_assert(NPW == 4, "a whole block or half of one");
       const W4 u = gload<W4>(b + 16 + 16 * pw + 32 * (q & 1) + 16 * (q >> 1));
       r.n[0] = u.x, r.n[1] = u.y, r.n[2] = u.z, r.n[3] = u.w;
-    } else {
-      const W2 u = gload<W2>(b + 16 + 16 * pw + 8 * q);
-      r.n[0] = u.x, r.n[1] = u.y;
     }
   }
   template <int NPW> struct H { uint32_t sc[2], mn[2]; float d, m; uint32_t n[NPW]; };
@@ -174,7 +172,7 @@ template <> struct Raw<kQ4_K> {
     if constexpr (NPW == 8) {  // lane: pair q, slots the four 8-byte units -> lane: unit q, slots the pairs
       swap1(h.n[0], h.n[4]), swap1(h.n[1], h.n[5]), swap1(h.n[2], h.n[6]), swap1(h.n[3], h.n[7]);
       swap0(h.n[0], h.n[2]), swap0(h.n[1], h.n[3]), swap0(h.n[4], h.n[6]), swap0(h.n[5], h.n[7]);
-    } else if constexpr (NPW == 4) {
+    } else {
       swap0(h.n[0], h.n[2]), swap0(h.n[1], h.n[3]);
     }
     h.sc[0] = hd[1] & 0x3F3F3F3Fu, h.mn[0] = hd[2] & 0x3F3F3F3Fu;
