@@ -9,7 +9,7 @@
 //
 // CDNA4 mapping: each step is v_mfma_f32_16x16x32_f16 (32 values: the gfx950 f16 MMA's K, the reference's WMMA takes
 // 16) - A the lane's row's 8 decoded values, B the same 8 columns of its token. Q4_0, Q3_K, Q4_K, IQ1_S, IQ1_M, IQ2_XXS and
-// IQ3_XXS decode straight from global memory (split_kernel, rows_kernel; mmraw.h); the other types, and a Q4_0 width that
+// IQ3_XXS decode straight from global memory (split_kernel, own_kernel, rows_kernel; mmraw.h); the other types, and a Q4_0 width that
 // is not whole 256s, stage their rows in LDS (kernel: a workgroup 16 rows x W waves, wave p partition p).
 #include <type_traits>
 

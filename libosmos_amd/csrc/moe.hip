@@ -540,7 +540,7 @@ inline bool aligned16(const void* a, const void* b, const void* c) { return (((u
 
 // ---- q4x_swiglu_rows (kernels/q4x_moe.hip:235-253): a thread 8 columns of a slot, silu(g) u (swiglu_kernel's expression)
 // rounded to f16 as mm_x16_rows rounds. Tiled: in x16's own order (mm.hip's x16_kernel), so that a wave stores side by side;
-// not for the few slots of up to two tiles, where a wave would hold few live threads (1 slot of 512: 3.1 us, 3.9 tiled). Vec: g
+// not for the few slots of up to two tiles, where a wave would hold few live threads (1 slot of 512: 2.7 us, 4.0 tiled). Vec: g
 // and u 16-byte aligned (7936 slots of 2048, 99 MB: 69 -> 22 us) ----
 template <bool Vec, bool Tiled>
 __global__ __launch_bounds__(256) void swiglu_rows_kernel(const float* __restrict__ g, const float* __restrict__ u,
