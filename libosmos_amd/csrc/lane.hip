@@ -608,7 +608,10 @@ bool tab_launch(const Args& a, hipStream_t s, bool* taken) {
 // IQ2_XXS 13.4 -> 14.5; 1024 x 1024 IQ2_XXS 13.4 -> 11.2; 2048 x 7168 IQ1_S 142 -> 51. full entries of 8 tokens: 8 of gate/up
 // 2048 x 7168 IQ2_XXS 97 -> 138, 8 of 512 x 2048 IQ1_S 11.0 -> 13.7, 64 of it 57 -> 83; few workgroups: q8_group_tok, 2 of
 // 2048 x 512 at 2 tokens, IQ1_S 2.8 -> 3.6. one token, 10 of 2048 x 2048: IQ3_XXS 17.2 -> 10.8, IQ1_S 9.1 -> 8.1, IQ2_XS 10.5 ->
-// 11.3 (9 of 7168 x 2048 26.5 -> 24.5); of 1024 x 1024 IQ1_M 4.5 -> 4.9
+// 11.3 (9 of 7168 x 2048 26.5 -> 24.5); of 1024 x 1024 IQ1_M 4.5 -> 4.9. gate/up at 2048 columns, more than 4 tokens, by workgroups,
+// tiles / per row: IQ2_XXS 4096 0.95, 11264 1.0, 21504 1.12, 22528 1.08, 57344 1.11; IQ2_S 4096 0.86, 21504 1.08, 57344 1.10; at
+// 1536 columns Q4_0 1.13 to 1.27 (at most 4 tokens 0.85), Q2_K 0.97 to 1.07. a dense table of more than 4 tokens an entry loses
+// by up to 1.3 to 1.9 where a sparse one of the same size wins by 0.7 to 0.9: the host cannot tell them apart
 template <uint32_t T, int L, int MATS>
 constexpr bool tabs_serve() { return T != kQ3_K ? !(T == kQ4_0 && MATS == 2 && L == 32) : MATS == 2 && L == 16; }
 template <uint32_t T, int L, int MATS>
@@ -621,7 +624,9 @@ bool tabs_pay(uint32_t n, uint32_t max_cnt, uint32_t rows, uint32_t cols, uint32
     if constexpr (T == kQ3_K) return cols > 1536 && (max_cnt <= 3 || (few && wgs <= 256));
     if constexpr (T == kIQ3_XXS || T == kQ4_K)
       return cols > (T == kQ4_K ? 1536 : 1024) || (cols >= 1024 && (few || some) && one_step);
-    return cols > (T == kQ2_K || T == kQ4_0 ? 1024 : 1536) && (few || routed) && (one_step || T == kIQ1_M || (T == kQ2_K && cols > 1536));
+    constexpr bool kIq12 = kIq && T != kIQ1_M;  // (the per-row kernels' loads of these suffice where the chip is full)
+    if (few) return cols > (T == kQ2_K || T == kQ4_0 ? 1024 : 1536) && (one_step || T == kIQ1_M || (T == kQ2_K && cols > 1536));
+    return cols > 1536 && routed && (!kIq12 || wgs <= 12288) && (one_step || T == kIQ1_M || T == kQ2_K);
   }
   if constexpr (MATS == 2) {
     if constexpr (kIq1) return max_cnt <= 3 || some;
